@@ -216,7 +216,11 @@ __global__ __launch_bounds__(256, 2) void shared_linear_kernel(
 // Large-tile path for bf16 activations with k % 64 == 0.
 //
 // Block tile 256x256 with eight waves, two per SIMD, in a 2 (m) x 4 (n) grid
-// of 128x64 wave tiles (4x2 MFMA 32x32x16 accumulators = 128 fp32 per lane).
+// of 128x64 wave tiles (8x4 MFMA 16x16x32 accumulators = 128 fp32 per lane).
+// 16x16x32 takes the same operand bytes from LDS as 32x32x16 and the same
+// matrix cycles, but moves half the accumulator registers per flop; under the
+// power limit that clocks higher: MLP up + down of the 720p video 1973 -> 1868
+// us, QKV projection + attention 988 -> 953 us.
 // The two waves of a SIMD ping-pong: one issues a whole 64-k step of MFMAs
 // from fragment registers while the other reads its next step's fragments
 // from LDS (the main loop below).  The operands stream through two 64-k LDS
@@ -329,12 +333,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
-    const int l32 = lane & 31;
-    const int g = lane >> 5;
+    const int l16 = lane & 15;
+    const int g = lane >> 4;
     const int wm = wave >> 2;
     const int wn = wave & 3;
     const int nk = k / BK;
-    const int sw = lds_swizzle(l32);   // fragment rows differ from l32 by multiples of 32
+    const int sw = lds_swizzle(l16);   // fragment rows differ from l16 by multiples of 16
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
 
     // The two token streams share one row space: video row r is row r, text
@@ -371,14 +375,16 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         }
     };
 
-    f32x16 acc[4][2];
+    // register r of accumulator [i][j] is row 16 i + 4 g + r, column 16 j + l16
+    // of the wave's 128x64 tile
+    f32x4 acc[8][4];
 
     // Thread coordinates for the epilogues, derived from an opaque copy of
     // the thread index: addresses computed from them are not hoisted above
     // the main loop, where every register is taken and hoisted values would
     // be spilled and reloaded one scratch round trip at a time.
     struct EpiIds {
-        int tid, l32, g, wm, wn;
+        int tid, l16, g, wm, wn;
     };
     auto epi_ids = [&]() {
         EpiIds e;
@@ -386,8 +392,8 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         asm volatile("" : "+v"(t));
         const int w = __builtin_amdgcn_readfirstlane(t >> 6);
         e.tid = t;
-        e.l32 = t & 31;
-        e.g = (t >> 5) & 1;
+        e.l16 = t & 15;
+        e.g = (t >> 4) & 3;
         e.wm = w >> 2;
         e.wn = w & 3;
         return e;
@@ -400,16 +406,16 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         if constexpr (YK != 0 && AWA == 0 && ACT != S2_ACT_SWIGLU) {
             const EpiIds ei = epi_ids();
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int cl = ei.wn * 64 + 32 * j + ei.l32;
+            for (int j = 0; j < 4; ++j) {
+                const int cl = ei.wn * 64 + 16 * j + ei.l16;
                 const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < 8; ++i)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
+                    for (int r = 0; r < 4; ++r) {
                         float v = acc[i][j][r] + bv;
                         if (ACT == S2_ACT_GELU) v = gelu(v);
-                        const int rl = ei.wm * 128 + 32 * i + 8 * (r >> 2) + 4 * ei.g + (r & 3);
+                        const int rl = ei.wm * 128 + 16 * i + 4 * ei.g + r;
                         if (YK == 2)
                             *(_Float16*)(lds + rl * EP + cl * 2) = f32_to_f16(v);
                         else
@@ -423,7 +429,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     //
     // Ping-pong main loop.  The two waves of each SIMD (wave w and w + 4:
     // group 0 owns tile rows 0-127, group 1 rows 128-255) take turns: one
-    // issues the 32 MFMAs of a whole 64-k step from fragment registers while
+    // issues the 64 MFMAs of a whole 64-k step from fragment registers while
     // the other reads its fragments of the next step from LDS, so the matrix
     // core never waits on an LDS read.  Every phase ends at a workgroup
     // barrier; group 1 runs one phase behind group 0.  The DMA of a step is
@@ -499,19 +505,19 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                           __builtin_amdgcn_readfirstlane(st + j * 1024), vo, soff);
             }
         };
-        bf16x8 fa[4][4], fb[4][2];
+        bf16x8 fa[2][8], fb[2][4];
         auto read_step = [&](int stage) {
             const uint8_t* st = lds + stage * SB;
 #pragma unroll
-            for (int kk = 0; kk < BK / 16; ++kk) {
-                const int pc = ((2 * kk + g) ^ sw) * 16;
+            for (int kk = 0; kk < BK / 32; ++kk) {
+                const int pc = ((4 * kk + g) ^ sw) * 16;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    fa[kk][i] = as_bf16x8(*(const uint4*)(st + (wm * 128 + 32 * i + l32) * RB + pc));
+                for (int i = 0; i < 8; ++i)
+                    fa[kk][i] = as_bf16x8(*(const uint4*)(st + (wm * 128 + 16 * i + l16) * RB + pc));
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+                for (int j = 0; j < 4; ++j)
                     fb[kk][j] =
-                        as_bf16x8(*(const uint4*)(st + TB + (wn * 64 + 32 * j + l32) * RB + pc));
+                        as_bf16x8(*(const uint4*)(st + TB + (wn * 64 + 16 * j + l16) * RB + pc));
             }
         };
         auto barrier = [] {
@@ -520,11 +526,9 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             __builtin_amdgcn_sched_barrier(0);
         };
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int steps = ke - kb;
         // steps 0 and 1: group 0 loads A, group 1 B
         issue(0, kb, grp);
@@ -546,12 +550,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             // MFMA phase
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int kk = 0; kk < BK / 16; ++kk)
+            for (int kk = 0; kk < BK / 32; ++kk)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < 8; ++i)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk][j],
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[kk][i], fb[kk][j],
                                                                             acc[i][j], 0, 0, 0);
             __builtin_amdgcn_s_setprio(0);
             if (grp == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // A of step s + 1
@@ -583,9 +587,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
 #pragma clang fp contract(off)
             constexpr int D = AWA;
             constexpr int SP = BN * 2 + 16;   // bytes per staged row
-            // transposed (v) staging: 8-byte writes of 32 lanes to 32 rows;
-            // a pitch of 130 dwords puts them on distinct bank pairs
-            constexpr int SPV = BN * 2 + 8;
+            // transposed (v) staging: 8-byte writes of 16 lanes to 16 rows,
+            // of the next 16 lanes beside them; a pitch of 132 dwords puts
+            // 32 lanes on distinct bank pairs
+            constexpr int SPV = BN * 2 + 16;
             // an opaque copy of the thread index: nothing the epilogue derives
             // from it is hoisted above the main loop, where every register is
             // taken
@@ -595,27 +600,25 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             const int hbase = (col0 - part * awa.inner) / D;
             __syncthreads();   // every wave is done reading the last stage
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int cl = ei.wn * 64 + 32 * j + ei.l32;
+            for (int j = 0; j < 4; ++j) {
+                const int cl = ei.wn * 64 + 16 * j + ei.l16;
                 const float bv = bias ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < 8; ++i) {
+                    // the four registers: rows rl .. rl + 3 of column cl
+                    const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
+                    uint16_t hv[4];
 #pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4) {
-                        // registers 4 q4 .. 4 q4 + 3: rows rl .. rl + 3 of column cl
-                        const int rl = ei.wm * 128 + 32 * i + 8 * q4 + 4 * ei.g;
-                        uint16_t hv[4];
+                    for (int e = 0; e < 4; ++e)
+                        hv[e] = __builtin_bit_cast(uint16_t, (__bf16)(acc[i][j][e] + bv));
+                    if (part < 2) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            hv[e] = __builtin_bit_cast(uint16_t, (__bf16)(acc[i][j][4 * q4 + e] + bv));
-                        if (part < 2) {
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) *(uint16_t*)(lds + (rl + e) * SP + cl * 2) = hv[e];
-                        } else {
-                            *(uint2*)(lds + cl * SPV + rl * 2) =
-                                make_uint2(hv[0] | ((uint32_t)hv[1] << 16), hv[2] | ((uint32_t)hv[3] << 16));
-                        }
+                        for (int e = 0; e < 4; ++e) *(uint16_t*)(lds + (rl + e) * SP + cl * 2) = hv[e];
+                    } else {
+                        *(uint2*)(lds + cl * SPV + rl * 2) =
+                            make_uint2(hv[0] | ((uint32_t)hv[1] << 16), hv[2] | ((uint32_t)hv[3] << 16));
                     }
+                }
             }
             __syncthreads();
             if (part < 2) {
@@ -771,14 +774,14 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 __syncthreads();   // the stage (h = 0) or the previous half is no longer read
                 if (ei.wm == h) {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int cl = ei.wn * 64 + 32 * j + ei.l32;
+                    for (int j = 0; j < 4; ++j) {
+                        const int cl = ei.wn * 64 + 16 * j + ei.l16;
                         const float bv = bias ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
+                        for (int i = 0; i < 8; ++i)
 #pragma unroll
-                            for (int r = 0; r < 16; ++r) {
-                                const int rl = 32 * i + 8 * (r >> 2) + 4 * ei.g + (r & 3);
+                            for (int r = 0; r < 4; ++r) {
+                                const int rl = 16 * i + 4 * ei.g + r;
                                 *(float*)(lds + rl * EF + cl * 4) = acc[i][j][r] + bv;
                             }
                     }
@@ -1019,16 +1022,16 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 __syncthreads();   // the stage (h = 0) or the previous half is no longer read
                 if (ei.wm == h) {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int cl = ei.wn * 64 + 32 * j + ei.l32;
+                    for (int j = 0; j < 4; ++j) {
+                        const int cl = ei.wn * 64 + 16 * j + ei.l16;
                         const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
+                        for (int i = 0; i < 8; ++i)
 #pragma unroll
-                            for (int r = 0; r < 16; ++r) {
+                            for (int r = 0; r < 4; ++r) {
                                 float v = acc[i][j][r] + bv;
                                 if (ACT == S2_ACT_GELU) v = gelu(v);
-                                const int rl = 32 * i + 8 * (r >> 2) + 4 * ei.g + (r & 3);
+                                const int rl = 16 * i + 4 * ei.g + r;
                                 *(float*)(lds + rl * EF + cl * 4) = v;
                             }
                     }
@@ -1049,18 +1052,17 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             }
             return;
         }
-        // ragged n: direct stores, register r of a 32x32 accumulator is row
-        // 8(r/4) + 4g + r%4, column l32
+        // ragged n: direct stores
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int col = col0 + ei.wn * 64 + 32 * j + ei.l32;
+        for (int j = 0; j < 4; ++j) {
+            const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
             if (col >= n) continue;
             const float bv = bias ? bias[col] : 0.f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    void* yr = out_row(ei.wm * 128 + 32 * i + 8 * (r >> 2) + 4 * ei.g + (r & 3));
+                for (int r = 0; r < 4; ++r) {
+                    void* yr = out_row(ei.wm * 128 + 16 * i + 4 * ei.g + r);
                     if (!yr) continue;
                     float v = acc[i][j][r] + bv;
                     if (ACT == S2_ACT_GELU) v = gelu(v);
@@ -1116,17 +1118,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             const __amdgpu_buffer_rsrc_t mine = __builtin_amdgcn_make_buffer_rsrc(
                 sk.slots + (long)s * kSlotFloats, (short)0, kSlotFloats * 4, kRawBufferFormat);
 #pragma unroll
-            for (int ii = 0; ii < 4; ++ii)
+            for (int ii = 0; ii < 8; ++ii)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        f32x4 v = {acc[ii][j][4 * c], acc[ii][j][4 * c + 1], acc[ii][j][4 * c + 2],
-                                   acc[ii][j][4 * c + 3]};
-                        __builtin_amdgcn_raw_buffer_store_b128(
-                            __builtin_bit_cast(u32x4, v), mine, tid * 16,
-                            ((ii * 2 + j) * 4 + c) * 512 * 16, kCoherent);
-                    }
+                for (int j = 0; j < 4; ++j)
+                    __builtin_amdgcn_raw_buffer_store_b128(
+                        __builtin_bit_cast(u32x4, acc[ii][j]), mine, tid * 16,
+                        (ii * 4 + j) * 512 * 16, kCoherent);
             // The slot stores write through to memory; every wave waits for
             // its own before the workgroup barrier.  The arrival is an
             // agent-scope acquire-release read-modify-write: it releases this
@@ -1145,44 +1142,33 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 // sum every part, this one's included, in workgroup order so
                 // that the result does not depend on the order of arrival
 #pragma unroll
-                for (int ii = 0; ii < 4; ++ii)
+                for (int ii = 0; ii < 8; ++ii)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[ii][j][r] = 0.f;
+                    for (int j = 0; j < 4; ++j) acc[ii][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
                 for (int q = lo; q <= hi; ++q) {
                     const __amdgpu_buffer_rsrc_t other = __builtin_amdgcn_make_buffer_rsrc(
                         sk.slots + (long)q * kSlotFloats, (short)0, kSlotFloats * 4, kRawBufferFormat);
-                    // sixteen 16-byte loads in flight per batch (four
+                    // sixteen 16-byte loads in flight per batch (sixteen
                     // accumulators; the fragment registers are free here)
 #pragma unroll
                     for (int h = 0; h < 2; ++h) {
                         __builtin_amdgcn_sched_barrier(0);
-                        f32x4 v[2][2][4];
+                        f32x4 v[4][4];
 #pragma unroll
-                        for (int iq = 0; iq < 2; ++iq)
+                        for (int iq = 0; iq < 4; ++iq)
 #pragma unroll
-                            for (int j = 0; j < 2; ++j)
+                            for (int j = 0; j < 4; ++j)
+                                v[iq][j] = __builtin_bit_cast(
+                                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                               other, tid * 16,
+                                               ((4 * h + iq) * 4 + j) * 512 * 16, kCoherent));
 #pragma unroll
-                                for (int c = 0; c < 4; ++c)
-                                    v[iq][j][c] = __builtin_bit_cast(
-                                        f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                   other, tid * 16,
-                                                   (((2 * h + iq) * 2 + j) * 4 + c) * 512 * 16,
-                                                   kCoherent));
+                        for (int iq = 0; iq < 4; ++iq)
 #pragma unroll
-                        for (int iq = 0; iq < 2; ++iq)
+                            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                                for (int c = 0; c < 4; ++c) {
-                                    f32x16& d = acc[2 * h + iq][j];
-                                    d[4 * c] += v[iq][j][c].x;
-                                    d[4 * c + 1] += v[iq][j][c].y;
-                                    d[4 * c + 2] += v[iq][j][c].z;
-                                    d[4 * c + 3] += v[iq][j][c].w;
-                                }
+                                for (int r = 0; r < 4; ++r) acc[4 * h + iq][j][r] += v[iq][j][r];
                     }
                 }
                 if (tid == 0)
