@@ -256,26 +256,29 @@ struct ConvArgs {
     int* counters;
 };
 
-// Epilogue of a TM x TN grid of 32x32 accumulators whose first row is GEMM
-// row r0 and first column output channel c0: register r of an accumulator
-// is row 8(r/4) + 4g + r%4, column l32, so each lane holds 4 consecutive
-// output pixels of one output channel: one 16-byte (fp32) or 8-byte store
-// into that plane.  part: the raw fp32 partial tile of k range blockIdx.y
-// goes to part + blockIdx.y * part_split (planar [cout][M]) instead.
-template <int TM, int TN, int OK>
-__device__ __forceinline__ void conv3d_epilogue(const ConvArgs& a, const f32x16 (&acc)[TM][TN],
-                                                int r0, int c0, int l32, int g, float* part) {
+// Epilogue of a TM x TN grid of square accumulators (f32x16: 32x32, f32x4:
+// 16x16) whose first row is GEMM row r0 and first column output channel c0:
+// register r of an accumulator is row 8(r/4) + 4g + r%4, column lcol, so each
+// lane holds 4 consecutive output pixels of one output channel: one 16-byte
+// (fp32) or 8-byte store into that plane.  part: the raw fp32 partial tile of
+// k range blockIdx.y goes to part + blockIdx.y * part_split (planar
+// [cout][M]) instead.
+template <int TM, int TN, int OK, typename Acc>
+__device__ __forceinline__ void conv3d_epilogue(const ConvArgs& a, const Acc (&acc)[TM][TN],
+                                                int r0, int c0, int lcol, int g, float* part) {
+    constexpr int QUADS = sizeof(Acc) / 16;      // 4-row runs a lane holds per accumulator
+    constexpr int SIDE = QUADS == 4 ? 32 : 16;   // accumulator rows and columns
     if (part) {
         float* pp = part + (long)blockIdx.y * a.part_split;
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const int col = c0 + 32 * j + l32;
+            const int col = c0 + SIDE * j + lcol;
             if (col >= a.cout) continue;
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int rg = 0; rg < 4; ++rg) {
-                    const int m = r0 + 32 * i + 8 * rg + 4 * g;
+                for (int rg = 0; rg < QUADS; ++rg) {
+                    const int m = r0 + SIDE * i + 8 * rg + 4 * g;
                     const long idx = (long)col * a.M + m;
                     if ((a.M & 3) == 0 && m + 3 < a.M) {
                         // m and M multiples of 4: a 16-byte aligned run
@@ -293,15 +296,15 @@ __device__ __forceinline__ void conv3d_epilogue(const ConvArgs& a, const f32x16 
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        const int col = c0 + 32 * j + l32;
+        const int col = c0 + SIDE * j + lcol;
         if (col >= a.cout) continue;
         const float bv = a.bias ? a.bias[col] : 0.f;
         const long cbase = (long)col * a.out_cstep + a.out_off;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-                const int m = r0 + 32 * i + 8 * rg + 4 * g;
+            for (int rg = 0; rg < QUADS; ++rg) {
+                const int m = r0 + SIDE * i + 8 * rg + 4 * g;
                 const float v0 = acc[i][j][4 * rg] + bv, v1 = acc[i][j][4 * rg + 1] + bv;
                 const float v2 = acc[i][j][4 * rg + 2] + bv, v3 = acc[i][j][4 * rg + 3] + bv;
                 if (a.vec_ok && m + 3 < a.M) {
@@ -583,10 +586,12 @@ __global__ __launch_bounds__(512, 1) void conv3d_kernel(ConvArgs a) {
 // window position and channel chunk, two LDS stages) with the SharedLinear
 // GEMM's main loop: the two waves of each SIMD (group 0 = waves 0-3, tile
 // rows 0-127; group 1 = waves 4-7, rows 128-255) take turns, one issuing the
-// 32 MFMAs of a whole 64-k step from fragment registers while the other
+// 64 MFMAs of a whole 64-k step from fragment registers while the other
 // reads its next step's fragments from LDS, so the matrix core does not wait
-// on LDS reads.  Every phase ends at a workgroup barrier; group 1 runs one
-// phase behind group 0.  Each wave loads A rows and B rows 128 grp + 32 wq
+// on LDS reads.  As in the GEMM the MFMAs are 16x16x32 (two slices of
+// 512-channel 90x160 frames: 394 us with 32x32x16, 371 us with these).
+// Every phase ends at a workgroup barrier; group 1 runs one phase behind
+// group 0.  Each wave loads A rows and B rows 128 grp + 32 wq
 // + 8 j + lane / 8 (j < 4) of a step, its group's half of the stage:
 //
 //   phase     2s                             2s + 1
@@ -616,9 +621,9 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2, wq = wave & 3;
-    const int l32 = lane & 31;
-    const int g = lane >> 5;
-    const int sw = lds_swizzle(l32);
+    const int l16 = lane & 15;
+    const int g = lane >> 4;
+    const int sw = lds_swizzle(l16);
     const uint32_t lds_base = (uint32_t)(uintptr_t)lds;
 
     const int lid = xcd_remap(blockIdx.x, gridDim.x);
@@ -729,19 +734,19 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
         }
     };
 
-    f32x16 acc[4][2];
-    bf16x8 fa[4][4], fb[4][2];
+    f32x4 acc[8][4];
+    bf16x8 fa[2][8], fb[2][4];
     auto read_step = [&](int stage) {
         const uint8_t* st = lds + stage * SB;
 #pragma unroll
-        for (int kk = 0; kk < BK / 16; ++kk) {
-            const int pc = ((2 * kk + g) ^ sw) * 16;
+        for (int kk = 0; kk < BK / 32; ++kk) {
+            const int pc = ((4 * kk + g) ^ sw) * 16;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                fa[kk][i] = as_bf16x8(*(const uint4*)(st + (grp * 128 + 32 * i + l32) * RB + pc));
+            for (int i = 0; i < 8; ++i)
+                fa[kk][i] = as_bf16x8(*(const uint4*)(st + (grp * 128 + 16 * i + l16) * RB + pc));
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-                fb[kk][j] = as_bf16x8(*(const uint4*)(st + TA + (wq * 64 + 32 * j + l32) * RB + pc));
+            for (int j = 0; j < 4; ++j)
+                fb[kk][j] = as_bf16x8(*(const uint4*)(st + TA + (wq * 64 + 16 * j + l16) * RB + pc));
         }
     };
     auto barrier = [] {
@@ -750,11 +755,9 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
         __builtin_amdgcn_sched_barrier(0);
     };
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // steps 0 and 1 by both groups
     issue(0);
@@ -776,12 +779,12 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
         // MFMA phase
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int kk = 0; kk < BK / 16; ++kk)
+        for (int kk = 0; kk < BK / 32; ++kk)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk][i], fb[kk][j],
+                for (int j = 0; j < 4; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[kk][i], fb[kk][j],
                                                                         acc[i][j], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
         if (grp == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // its half of step s + 1
@@ -803,17 +806,11 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
         };
         const __amdgpu_buffer_rsrc_t mine = slot((int)blockIdx.y);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    const f32x4 v = {acc[i][j][4 * c], acc[i][j][4 * c + 1], acc[i][j][4 * c + 2],
-                                     acc[i][j][4 * c + 3]};
-                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), mine,
-                                                           tid * 16, ((i * 2 + j) * 4 + c) * 512 * 16,
-                                                           kFlags);
-                }
+            for (int j = 0; j < 4; ++j)
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[i][j]), mine,
+                                                       tid * 16, (i * 4 + j) * 512 * 16, kFlags);
         __shared__ int arrival;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -833,44 +830,31 @@ __global__ __launch_bounds__(512, 1) void conv3d_pp_kernel(ConvArgs a) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 __builtin_amdgcn_sched_barrier(0);
-                f32x4 v[2][2][4];
+                f32x4 v[4][4];
 #pragma unroll
-                for (int iq = 0; iq < 2; ++iq)
+                for (int iq = 0; iq < 4; ++iq)
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
+                    for (int j = 0; j < 4; ++j)
+                        v[iq][j] = __builtin_bit_cast(
+                            f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                       other, tid * 16, ((4 * h + iq) * 4 + j) * 512 * 16, kFlags));
 #pragma unroll
-                        for (int c = 0; c < 4; ++c)
-                            v[iq][j][c] = __builtin_bit_cast(
-                                f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                           other, tid * 16, (((2 * h + iq) * 2 + j) * 4 + c) * 512 * 16,
-                                           kFlags));
+                for (int iq = 0; iq < 4; ++iq)
 #pragma unroll
-                for (int iq = 0; iq < 2; ++iq)
+                    for (int j = 0; j < 4; ++j) {
+                        f32x4& d = acc[4 * h + iq][j];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) {
-                            f32x16& d = acc[2 * h + iq][j];
-                            if (r == 0 && !two) {
-                                d[4 * c] = v[iq][j][c].x;
-                                d[4 * c + 1] = v[iq][j][c].y;
-                                d[4 * c + 2] = v[iq][j][c].z;
-                                d[4 * c + 3] = v[iq][j][c].w;
-                            } else {
-                                d[4 * c] += v[iq][j][c].x;
-                                d[4 * c + 1] += v[iq][j][c].y;
-                                d[4 * c + 2] += v[iq][j][c].z;
-                                d[4 * c + 3] += v[iq][j][c].w;
-                            }
-                        }
+                        for (int e = 0; e < 4; ++e)
+                            d[e] = r == 0 && !two ? v[iq][j][e] : d[e] + v[iq][j][e];
+                    }
             }
         }
         if (tid == 0)
             __hip_atomic_store(&a.counters[tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        conv3d_epilogue<4, 2, OK>(a, acc, row0 + 128 * grp, col0 + 64 * wq, l32, g, nullptr);
+        conv3d_epilogue<8, 4, OK>(a, acc, row0 + 128 * grp, col0 + 64 * wq, l16, g, nullptr);
         return;
     }
-    conv3d_epilogue<4, 2, OK>(a, acc, row0 + 128 * grp, col0 + 64 * wq, l32, g, a.part);
+    conv3d_epilogue<8, 4, OK>(a, acc, row0 + 128 * grp, col0 + 64 * wq, l16, g, a.part);
 }
 
 // ---- 3x3 spatial windows, stride 1: the halo kernel --------------------------
