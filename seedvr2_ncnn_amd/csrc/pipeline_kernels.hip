@@ -64,12 +64,19 @@ __global__ void __launch_bounds__(kThreads) latent_patches_kernel(
     const int tid = threadIdx.x;
     const int col = tid & 63;
     const long col0 = 2L * px0;
-#pragma unroll 4
-    for (int cy = tid >> 6; cy < 64; cy += 4) {
-        const int c = cy >> 1, y = cy & 1;
+    // a thread's sixteen loads are all in flight before the first is used
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int cy = (tid >> 6) + 4 * i, c = cy >> 1, y = cy & 1;
         const float* plane = c < 16 ? latent + c * cstride : condition + (c - 16) * cstride;
         const long tok = (2L * prow + y) * width + col0 + col;
-        if (col < ncol) tile[(y * 64 + col) * 33 + c] = plane[tok];
+        v[i] = col < ncol ? plane[tok] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int cy = (tid >> 6) + 4 * i, c = cy >> 1, y = cy & 1;
+        tile[(y * 64 + col) * 33 + c] = v[i];
     }
     if (tid < 128) tile[tid * 33 + 32] = 1.f;
     __syncthreads();
@@ -126,10 +133,16 @@ __global__ void __launch_bounds__(128) timestep_kernel(Timesteps ts, float* __re
 //
 // cfg = neg + scale (pos - neg).  With rescale, cfg *= (float)(rescale
 // std(pos)/std(cfg) + (1 - rescale)), the sample standard deviations over all
-// elements, unless std(cfg) is 0.  The statistics pass keeps, per block, the
-// count, mean and sum of squared deviations (M2) of pos and cfg in fp64 and
-// merges chunks and blocks with the pairwise update of Chan et al.: the same
-// two-pass quantities as the reference's, summed in another order.
+// elements, unless std(cfg) is 0.  The statistics pass writes, per block, the
+// count, mean and sum of squared deviations (M2) of pos and cfg in fp64 (waves
+// and blocks joined with the update of Chan et al.): the same two-pass
+// quantities as the reference's, summed in another order.  Every block of the
+// pass that scales joins the records itself, in one fixed order.
+//
+// Both passes are bound by latency, not by their 11 to 17 MB.  With a last
+// block of the statistics pass that merged the records in a tree of fp64
+// divisions behind an agent-scope counter, the statistics pass took 16.2 us at
+// the 720p latent (86,400 tokens) and the update 6.0; now they take 6.7 and 8.6.
 
 constexpr int kStatChunk = 4096;           // elements per block iteration, 16 per thread
 constexpr int kMaxStatBlocks = 1024;
@@ -155,9 +168,7 @@ __device__ __forceinline__ void merge(Moments& a, const Moments& b) {
 }
 
 struct CfgScratch {
-    Moments rec[kMaxStatBlocks];
-    int arrivals;       // blocks of the running statistics pass; 0 between launches
-    float factor[2];    // {factor, 1 = apply / 0 = leave cfg unscaled}
+    Moments rec[kMaxStatBlocks];   // one per block of the statistics pass
 };
 
 __device__ __forceinline__ float cfg_value(float p, float n, float scale) {
@@ -165,13 +176,18 @@ __device__ __forceinline__ float cfg_value(float p, float n, float scale) {
     return n + scale * (p - n);
 }
 
-// Sum of two doubles over the block, the same value in every thread.
-__device__ __forceinline__ void block_sum2(double& a, double& b, double* red) {
+// Sum of two doubles over the wave, the same value in every lane.
+__device__ __forceinline__ void wave_sum2(double& a, double& b) {
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) {
         a += __shfl_xor(a, m);
         b += __shfl_xor(b, m);
     }
+}
+
+// Sum of two doubles over the block, the same value in every thread.
+__device__ __forceinline__ void block_sum2(double& a, double& b, double* red) {
+    wave_sum2(a, b);
     const int wave = threadIdx.x >> 6;
     __syncthreads();   // red[] is free (its last readers are past this barrier)
     if ((threadIdx.x & 63) == 0) {
@@ -184,16 +200,14 @@ __device__ __forceinline__ void block_sum2(double& a, double& b, double* red) {
 }
 
 // Pass 1: cfg (stored when out is non-null) and the moments of pos and cfg.
-// The last block to finish merges the per-block moments in block order and
-// writes the factor.
+// A wave takes the moments of its part of a chunk around its own mean (no
+// barrier between the two sums); the four waves' moments join once, at the end.
 __global__ void __launch_bounds__(kThreads) cfg_stats_kernel(const float* __restrict__ pos,
                                                              const float* __restrict__ neg,
-                                                             long count, float scale, float rescale,
+                                                             long count, float scale,
                                                              float* __restrict__ out,
                                                              CfgScratch* sc) {
-    __shared__ double red[8];
-    __shared__ Moments all[kThreads];
-    __shared__ int last;
+    __shared__ Moments waves[kThreads / 64];
     const int tid = threadIdx.x;
     const long chunks = (count + kStatChunk - 1) / kStatChunk;
     Moments acc = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -234,9 +248,14 @@ __global__ void __launch_bounds__(kThreads) cfg_stats_kernel(const float* __rest
                 sp += (double)p[e];
                 sg += (double)g[e];
             }
-        block_sum2(sp, sg, red);
-        const double n = (double)min((long)kStatChunk, count - base);
-        const double mp = sp / n, mg = sg / n;
+        wave_sum2(sp, sg);
+        // elements of this wave: four runs of 256, those below count
+        long n = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            n += min(max(count - (base + j * 1024 + (tid >> 6) * 256), 0L), 256L);
+        const double inv = 1.0 / (double)max(n, 1L);
+        const double mp = sp * inv, mg = sg * inv;
         double qp = 0.0, qg = 0.0;
 #pragma unroll
         for (int e = 0; e < 16; ++e)
@@ -245,40 +264,55 @@ __global__ void __launch_bounds__(kThreads) cfg_stats_kernel(const float* __rest
                 qp += dp * dp;
                 qg += dg * dg;
             }
-        block_sum2(qp, qg, red);
-        merge(acc, Moments{n, mp, qp, mg, qg});
+        wave_sum2(qp, qg);
+        merge(acc, Moments{(double)n, mp, qp, mg, qg});
     }
+    if ((tid & 63) == 0) waves[tid >> 6] = acc;
+    __syncthreads();
     if (tid == 0) {
+#pragma unroll
+        for (int w = 1; w < kThreads / 64; ++w) merge(acc, waves[w]);
         sc->rec[blockIdx.x] = acc;
-        // release: the record is visible device-wide before the arrival counts
-        const int before = __hip_atomic_fetch_add(&sc->arrivals, 1, __ATOMIC_ACQ_REL,
-                                                  __HIP_MEMORY_SCOPE_AGENT);
-        last = before == (int)gridDim.x - 1;
     }
-    __syncthreads();
-    if (!last) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    Moments m = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int b = tid; b < (int)gridDim.x; b += kThreads) merge(m, sc->rec[b]);
-    all[tid] = m;
-    __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1) {
-        if (tid < s) merge(all[tid], all[tid + s]);
-        __syncthreads();
+}
+
+// The factor of the statistics' `nrec` records, the same value in every
+// thread of every block that asks: means around the first record's, then the
+// squared deviations around the joint mean.  Returns false when std(cfg) is 0
+// (the prediction stays unscaled).
+__device__ __forceinline__ bool cfg_factor(const CfgScratch* sc, int nrec, long count,
+                                           float rescale, double* red, float* factor) {
+    constexpr int PER = kMaxStatBlocks / kThreads;
+    Moments m[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int b = i * kThreads + (int)threadIdx.x;
+        m[i] = b < nrec ? sc->rec[b] : Moments{0.0, 0.0, 0.0, 0.0, 0.0};
     }
-    if (tid == 0) {
-        const double denom = (double)(count - 1);
-        const double pos_std = sqrt(all[0].qp / denom);
-        const double cfg_std = sqrt(all[0].qc / denom);
-        float factor = 1.f, apply = 0.f;
-        if (!(cfg_std == 0.0)) {
-            factor = (float)((double)rescale * pos_std / cfg_std + (double)(1.f - rescale));
-            apply = 1.f;
+    const double p0 = sc->rec[0].mp, c0 = sc->rec[0].mc;
+    double sp = 0.0, sg = 0.0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (m[i].n != 0.0) {
+            sp += m[i].n * (m[i].mp - p0);
+            sg += m[i].n * (m[i].mc - c0);
         }
-        sc->factor[0] = factor;
-        sc->factor[1] = apply;
-        __hip_atomic_store(&sc->arrivals, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    block_sum2(sp, sg, red);
+    const double mp = p0 + sp / (double)count, mc = c0 + sg / (double)count;
+    double qp = 0.0, qc = 0.0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        if (m[i].n != 0.0) {
+            const double dp = m[i].mp - mp, dc = m[i].mc - mc;
+            qp += m[i].qp + m[i].n * dp * dp;
+            qc += m[i].qc + m[i].n * dc * dc;
+        }
+    block_sum2(qp, qc, red);
+    const double denom = (double)(count - 1);
+    const double pos_std = sqrt(qp / denom);
+    const double cfg_std = sqrt(qc / denom);
+    *factor = (float)((double)rescale * pos_std / cfg_std + (double)(1.f - rescale));
+    return !(cfg_std == 0.0);
 }
 
 __global__ void __launch_bounds__(kThreads) cfg_kernel(const float* __restrict__ pos,
@@ -298,13 +332,16 @@ __global__ void __launch_bounds__(kThreads) cfg_kernel(const float* __restrict__
 
 // Pass 2 of apply_cfg: cfg *= factor, skipped when std(cfg) was 0.
 __global__ void __launch_bounds__(kThreads) cfg_scale_kernel(float* __restrict__ out, long count,
-                                                             const float* __restrict__ factor) {
+                                                             const CfgScratch* sc, int nrec,
+                                                             float rescale) {
 #pragma clang fp contract(off)
-    if (factor[1] == 0.f) return;
-    const float f = factor[0];
+    __shared__ double red[8];
     const long i = ((long)blockIdx.x * kThreads + threadIdx.x) * 4;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (i + 3 < count) v = *reinterpret_cast<const float4*>(out + i);
+    float f;
+    if (!cfg_factor(sc, nrec, count, rescale, red, &f)) return;
     if (i + 3 < count) {
-        float4 v = *reinterpret_cast<const float4*>(out + i);
         v.x *= f, v.y *= f, v.z *= f, v.w *= f;
         *reinterpret_cast<float4*>(out + i) = v;
     } else {
@@ -355,25 +392,45 @@ __global__ void __launch_bounds__(kThreads) euler_kernel(float* __restrict__ lat
 // factor, step = delta * cfg, latent += step.
 __global__ void __launch_bounds__(kThreads) denoise_update_kernel(
     const float* __restrict__ pos, const float* __restrict__ neg, float scale,
-    const float* __restrict__ factor, float delta, float* __restrict__ latent, long cstride,
-    int width, int pw, int tiles_per_row) {
+    const CfgScratch* sc, int nrec, long count, float rescale, float delta,
+    float* __restrict__ latent, long cstride, int width, int pw, int tiles_per_row) {
 #pragma clang fp contract(off)
     __shared__ float tile[2 * 64 * 17];
+    __shared__ double red[8];
     const int prow = blockIdx.x / tiles_per_row;
     const int px0 = (blockIdx.x - prow * tiles_per_row) * kTilePatches;
     const int npatch = min(kTilePatches, pw - px0);
     const int tid = threadIdx.x;
-    const bool scaled = factor && factor[1] != 0.f;
-    const float f = factor ? factor[0] : 1.f;
     const long pbase = ((long)prow * pw + px0) * 64;
+    // every load of the block goes out before the factor is formed
+    const int col = tid & 63;
+    const long colg = 2L * px0 + col;
+    float4 pv[2], nv[2];
+    float lat[8];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int e = (j * kThreads + tid) * 4;   // element of the block's [32][64]
+        pv[j] = nv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if ((e >> 6) < npatch) {
+            pv[j] = *reinterpret_cast<const float4*>(pos + pbase + e);
+            if (neg) nv[j] = *reinterpret_cast<const float4*>(neg + pbase + e);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int cy = (tid >> 6) + 4 * i, c = cy >> 1, y = cy & 1;
+        lat[i] = col < 2 * npatch ? latent[c * cstride + (2L * prow + y) * width + colg] : 0.f;
+    }
+    float f = 1.f;
+    const bool scaled = sc && cfg_factor(sc, nrec, count, rescale, red, &f);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int e = (j * kThreads + tid) * 4;
         const int p = e >> 6, rem = e & 63;
         if (p < npatch) {
-            float4 v = *reinterpret_cast<const float4*>(pos + pbase + e);
+            float4 v = pv[j];
             if (neg) {
-                const float4 b = *reinterpret_cast<const float4*>(neg + pbase + e);
+                const float4 b = nv[j];
                 v = make_float4(cfg_value(v.x, b.x, scale), cfg_value(v.y, b.y, scale),
                                 cfg_value(v.z, b.z, scale), cfg_value(v.w, b.w, scale));
                 if (scaled) v.x *= f, v.y *= f, v.z *= f, v.w *= f;
@@ -385,15 +442,12 @@ __global__ void __launch_bounds__(kThreads) denoise_update_kernel(
         }
     }
     __syncthreads();
-    const int col = tid & 63;
     if (col >= 2 * npatch) return;
-    const long colg = 2L * px0 + col;
 #pragma unroll
-    for (int cy = tid >> 6; cy < 32; cy += 4) {
-        const int c = cy >> 1, y = cy & 1;
-        float* dst = latent + c * cstride + (2L * prow + y) * width + colg;
+    for (int i = 0; i < 8; ++i) {
+        const int cy = (tid >> 6) + 4 * i, c = cy >> 1, y = cy & 1;
         const float step = delta * tile[(y * 64 + col) * 17 + c];
-        *dst = *dst + step;
+        latent[c * cstride + (2L * prow + y) * width + colg] = lat[i] + step;
     }
 }
 
@@ -405,11 +459,15 @@ hipError_t cfg_scratch(hipStream_t stream, CfgScratch** out) {
     return stream_scratch(kScratchCfg, stream, sizeof(CfgScratch), (void**)out);
 }
 
-hipError_t launch_stats(const float* pos, const float* neg, long count, float scale, float rescale,
-                        float* out, CfgScratch* sc, hipStream_t stream) {
-    const long chunks = (count + kStatChunk - 1) / kStatChunk;
-    const unsigned grid = (unsigned)min(chunks, (long)kMaxStatBlocks);
-    cfg_stats_kernel<<<grid, kThreads, 0, stream>>>(pos, neg, count, scale, rescale, out, sc);
+// records the statistics pass leaves: one per block
+int stat_blocks(long count) {
+    return (int)min((count + kStatChunk - 1) / kStatChunk, (long)kMaxStatBlocks);
+}
+
+hipError_t launch_stats(const float* pos, const float* neg, long count, float scale, float* out,
+                        CfgScratch* sc, hipStream_t stream) {
+    cfg_stats_kernel<<<(unsigned)stat_blocks(count), kThreads, 0, stream>>>(pos, neg, count, scale,
+                                                                           out, sc);
     return hipGetLastError();
 }
 
@@ -481,9 +539,9 @@ hipError_t launch_cfg(const float* pos, const float* neg, long count, float scal
     CfgScratch* sc = nullptr;
     hipError_t e = cfg_scratch(stream, &sc);
     if (e != hipSuccess) return e;
-    e = launch_stats(pos, neg, count, scale, rescale, out, sc, stream);
+    e = launch_stats(pos, neg, count, scale, out, sc, stream);
     if (e != hipSuccess) return e;
-    cfg_scale_kernel<<<grid, kThreads, 0, stream>>>(out, count, sc->factor);
+    cfg_scale_kernel<<<grid, kThreads, 0, stream>>>(out, count, sc, stat_blocks(count), rescale);
     return hipGetLastError();
 }
 
@@ -503,19 +561,17 @@ hipError_t launch_denoise_update(const float* pos_patches, const float* neg_patc
     const long tpr = (pw + kTilePatches - 1) / kTilePatches;
     if (prows == 0 || pw == 0) return hipSuccess;
     if (!fits_int(prows * tpr)) return hipErrorInvalidValue;
-    const float* factor = nullptr;
+    CfgScratch* sc = nullptr;
     const long count = prows * pw * 64;
     if (neg_patches && rescale != 0.f && count >= 2) {
-        CfgScratch* sc = nullptr;
         hipError_t e = cfg_scratch(stream, &sc);
         if (e != hipSuccess) return e;
-        e = launch_stats(pos_patches, neg_patches, count, scale, rescale, nullptr, sc, stream);
+        e = launch_stats(pos_patches, neg_patches, count, scale, nullptr, sc, stream);
         if (e != hipSuccess) return e;
-        factor = sc->factor;
     }
     denoise_update_kernel<<<(unsigned)(prows * tpr), kThreads, 0, stream>>>(
-        pos_patches, neg_patches, scale, factor, delta, latent, channel_stride, width, pw,
-        (int)tpr);
+        pos_patches, neg_patches, scale, sc, stat_blocks(count), count, rescale, delta, latent,
+        channel_stride, width, pw, (int)tpr);
     return hipGetLastError();
 }
 
