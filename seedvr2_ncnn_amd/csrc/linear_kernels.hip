@@ -309,7 +309,8 @@ struct AwaQkvArgs {
     uint16_t* vt;
 };
 
-template <int YK, int ACT, int AWA = 0, int RES = 0>
+// XK is the element type of x0 and x1 (0 fp32, 1 bf16, 2 fp16).
+template <int YK, int ACT, int AWA = 0, int RES = 0, int XK = 1>
 __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     const uint16_t* __restrict__ x0, int m0, const uint16_t* __restrict__ x1, int m1,
     const uint16_t* __restrict__ wgt, const float* __restrict__ bias, int n, int k,
@@ -564,6 +565,166 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         // group 0's barrier matching group 1's last MFMA phase; with an early
         // epilogue group 0 stages its rows first (epilogue)
         if (grp == 0 && !early) barrier();
+    };
+
+    // The same sum for fp32 and fp16 activations (XK != 1), which are rounded
+    // to bf16 (nearest even) between global memory and LDS.
+    //
+    // The DMA cannot convert, so A passes through registers: 32-k steps halve
+    // the fragments (48 registers) and leave room for two steps of A in flight
+    // (2 x 16 registers of fp32).  Lane l of wave w loads four consecutive k
+    // (chunk l % 8) of rows 32 w + l / 8 + 8 i, whole 128-byte lines for fp32,
+    // and writes them as 8 bytes of LDS; B comes by DMA.  Four 32 KB stages of
+    // 64-byte rows, 16-byte chunk c of row r at position c ^ ((r >> 2) & 3):
+    // a read phase covers rows that share banks only four apart.  The groups
+    // ping-pong as above, a phase being 32 k:
+    //
+    //   memory phase of step s   read step s; write A of step s + 2 (loaded
+    //                            two steps ago) and DMA B of step s + 2 into
+    //                            stage (s + 2) % 4, read last in step s - 2;
+    //                            load A of step s + 4; wait for B of step s + 1
+    //
+    // 3677 x 2560 by 2560 x 2560 from fp32: 104 us (150 tiles on 256 CUs), 262 us
+    // with the 128 kernel, which staged A through registers one step ahead and
+    // rounded it with integer operations; 15064 x 3072 by 9216 x 3072 from fp32
+    // 1074 against 2775 us, 1038 us from fp16, 272 x 2560 by 2560 x 2560 50
+    // against 131 us.
+    auto mainloop_cvt = [&](int kb, int ke) {
+        if constexpr (XK != 1) {
+        constexpr int ES = XK == 0 ? 4 : 2;      // bytes per activation
+        constexpr int SBC = 2 * 256 * 64;        // stage bytes: A, then B
+        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+        typedef typename std::conditional<XK == 0, u32x4, u32x2>::type Raw;   // four k
+        const int grp = wave >> 2;
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+            (char*)x0 + (long)row0 * k * ES, (short)0, max(min(m0 - row0, BM), 0) * k * ES,
+            kRawBufferFormat);
+        const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(
+            (char*)x1 + (long)(row0 - mv) * k * ES, (short)0,
+            row0 + BM > mv ? min(mv + m1 - row0, BM) * k * ES : 0, kRawBufferFormat);
+        const i32x4 rb =
+            wave_uniform(buffer_rsrc(wgt + (long)col0 * k, (uint32_t)(min(n - col0, BN) * k * 2)));
+        const int wrow = __builtin_amdgcn_readfirstlane(row0 + wave * 32);
+        const int arow = wave * 32 + (lane >> 3);
+        const uint32_t aoff = (uint32_t)(arow * k * ES + (lane & 7) * 4 * ES);
+        // LDS bytes of the lane's chunk in row arow; rows 8 apart differ in
+        // bit 1 of the swizzle
+        const uint32_t awr = (uint32_t)(arow * 64 + ((((lane & 7) >> 1) ^ ((arow >> 2) & 3)) << 4) +
+                                        (lane & 1) * 8);
+        const int brow = wave * 32 + (lane >> 2);
+        const uint32_t boff = (uint32_t)(brow * k * 2 + (((lane & 3) ^ ((lane >> 4) & 3)) * 16));
+        auto load_a = [&](int kt, Raw (&raw)[4]) {
+            const int soff = __builtin_amdgcn_readfirstlane(kt * 32 * ES);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int vo = (int)aoff + i * 8 * k * ES;
+                if constexpr (XK == 0) {
+                    if (wrow + 8 * i < mv)
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rv, vo, soff, 0);
+                    else
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b128(rt, vo, soff, 0);
+                } else {
+                    if (wrow + 8 * i < mv)
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b64(rv, vo, soff, 0);
+                    else
+                        raw[i] = __builtin_amdgcn_raw_buffer_load_b64(rt, vo, soff, 0);
+                }
+            }
+        };
+        auto write_a = [&](int stage, const Raw (&raw)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float f[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (XK == 0)
+                        f[e] = __uint_as_float(raw[i][e]);
+                    else
+                        f[e] = (float)__builtin_bit_cast(_Float16, (uint16_t)(raw[i][e >> 1] >> (16 * (e & 1))));
+                }
+                *(uint2*)(lds + stage * SBC + i * 512 + (awr ^ ((i & 1) << 5))) =
+                    make_uint2(pack2_bf16_rne(f[0], f[1]), pack2_bf16_rne(f[2], f[3]));
+            }
+        };
+        auto dma_b = [&](int stage, int kt) {
+            const uint32_t soff = __builtin_amdgcn_readfirstlane((uint32_t)(kt * 64));
+            const uint32_t st = lds_base + stage * SBC + SBC / 2 + wave * 32 * 64;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                lds_dma16(rb, __builtin_amdgcn_readfirstlane(st + j * 1024),
+                          boff + (uint32_t)(j * 16 * k * 2), soff);
+        };
+        bf16x8 fa[8], fb[4];
+        const int pc = ((g ^ (l16 >> 2)) & 3) * 16;
+        auto barrier = [] {
+            __builtin_amdgcn_sched_barrier(0);
+            asm volatile("s_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int steps = 2 * (ke - kb);   // even, at least 2
+        const int k0 = 2 * kb;
+        Raw ra0[4], ra1[4];   // A of the next even and odd step to write
+        {
+            Raw p0[4], p1[4];
+            load_a(k0, p0);
+            load_a(k0 + 1, p1);
+            dma_b(0, k0);
+            dma_b(1, k0 + 1);
+            if (steps > 2) {
+                load_a(k0 + 2, ra0);
+                load_a(k0 + 3, ra1);
+            }
+            write_a(0, p0);
+            write_a(1, p1);
+            if (steps > 2)
+                asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // B of steps 0 and 1
+            else
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+        barrier();
+        if (grp == 1) barrier();
+        auto step = [&](int s, Raw (&raw)[4]) {
+            const uint8_t* st = lds + (s & 3) * SBC;
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                fa[i] = as_bf16x8(*(const uint4*)(st + (wm * 128 + 16 * i + l16) * 64 + pc));
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                fb[j] = as_bf16x8(*(const uint4*)(st + SBC / 2 + (wn * 64 + 16 * j + l16) * 64 + pc));
+            if (s + 2 < steps) {
+                write_a((s + 2) & 3, raw);
+                dma_b((s + 2) & 3, k0 + s + 2);
+                if (s + 4 < steps) load_a(k0 + s + 4, raw);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            // B of step s + 1: in flight behind it are A of step s + 3, B of
+            // step s + 2 and A of step s + 4
+            if (s + 4 < steps)
+                asm volatile("s_waitcnt vmcnt(10)" ::: "memory");
+            else
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            barrier();
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_s_setprio(0);
+            barrier();
+        };
+#pragma unroll 1
+        for (int s = 0; s < steps; s += 2) {
+            step(s, ra0);
+            step(s + 1, ra1);
+        }
+        if (grp == 0) barrier();
+        }
     };
 
     // Fused QKV epilogue.  The tile's 256 columns lie in one of q, k, v
@@ -1109,9 +1270,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         // the plain 16-bit epilogue of a whole tile without an activation runs
         // early (see epilogue); with GELU the early schedule would serialise
         // the two groups' VALU work, which otherwise shares the SIMDs
-        const bool early = AWA == 0 && RES == 0 && ACT == S2_ACT_NONE && YK != 0 &&
+        const bool early = AWA == 0 && RES == 0 && XK == 1 && ACT == S2_ACT_NONE && YK != 0 &&
                            (n & 7) == 0 && finish;
-        mainloop(kb, ke, early);
+        if constexpr (XK == 1)
+            mainloop(kb, ke, early);
+        else
+            mainloop_cvt(kb, ke);
         if (!finish) {
             // slot layout: float4 c (4 accumulator registers) of thread tid
             // at byte (c * 512 + tid) * 16; the chunk index goes in soffset
@@ -1369,11 +1533,11 @@ template <typename TX, int YK, int ACT>
 static hipError_t linear_impl(const void* x0, int m0, const void* x1, int m1, const uint16_t* w,
                               const float* bias, int n, int k, void* y0, void* y1,
                               hipStream_t stream, SkSource source) {
-    // bf16 activations (the operand type of the MFMAs) go straight to LDS;
-    // fp32 and fp16 ones are rounded to bf16 while staged by the 128 kernel
-    if (std::is_same<TX, uint16_t>::value && k % 64 == 0 &&
-        (long)256 * k * 2 <= 0x7fffffffL &&   // buffer offsets are 32-bit
+    // k that is no multiple of the 64-k step, and tiles beyond the buffers'
+    // 32-bit offsets, take the 128 kernel
+    if (k % 64 == 0 && (long)256 * k * (long)sizeof(TX) <= 0x7fffffffL &&
         (long)256 * n * 4 <= 0x7fffffffL) {
+        constexpr int XK = std::is_same<TX, float>::value ? 0 : std::is_same<TX, uint16_t>::value ? 1 : 2;
         const int mv = (m0 + 7) / 8 * 8;   // first text row in the joint row space
         const int ntiles = (n + 255) / 256;
         const int mtiles = (mv + m1 + 255) / 256;
@@ -1383,7 +1547,7 @@ static hipError_t linear_impl(const void* x0, int m0, const void* x1, int m1, co
         hipError_t e = plan_sk_tail(tiles, k / 64, source, stream, &sk);
         if (e != hipSuccess) return e;
         const long blocks = (long)sk.dp_tiles + sk.sk_groups;
-        shared_linear_256_kernel<YK, ACT><<<(unsigned)blocks, 512, 0, stream>>>(
+        shared_linear_256_kernel<YK, ACT, 0, 0, XK><<<(unsigned)blocks, 512, 0, stream>>>(
             (const uint16_t*)x0, m0, (const uint16_t*)x1, m1, w, bias, n, k, y0, y1, mv, mtiles,
             ntiles, sk, AwaQkvArgs{}, LinearResidual{});
         return hipGetLastError();

@@ -1,0 +1,34 @@
+"""fp32 and fp16 activations on the 256-tile GEMM (k a multiple of 64): the
+kernel rounds them to bf16 between global memory and LDS and then adds the
+same 32-k products in the same order as for bf16 activations, so the result
+equals, bit for bit, that of the rounded activations given as bf16 (which
+tests/test_gpu_linear.py checks against the oracle)."""
+import pytest
+
+from seedvr2_ncnn_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+# one row; a video tail off an 8-row group with text rows in its tile; two,
+# four and six 32-k steps (the pipeline's start and end); ragged n (direct
+# stores); a split tail; rows past two tiles
+CASES = [(1, 0, 64, 64), (37, 5, 128, 40), (250, 70, 192, 260), (257, 3, 64, 512),
+         (300, 40, 2560, 1000), (600, 1, 1088, 2560)]
+
+
+@pytest.mark.parametrize("mv,mt,k,n", CASES)
+@pytest.mark.parametrize("act", [capi.ACT_NONE, capi.ACT_GELU])
+def test_equals_the_rounded_activations_as_bf16(mv, mt, k, n, act):
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(mv + k)
+    draw = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    xv, xt = draw(mv, k), draw(mt, k) if mt else None
+    w, b = (0.02 * draw(n, k)).bfloat16(), 0.02 * draw(n)
+    for dt in (torch.float32, torch.float16):
+        v, t = xv.to(dt), xt.to(dt) if mt else None
+        got = capi.shared_linear(v, t, w, b, act, out_dtype=torch.float32)
+        ref = capi.shared_linear(v.bfloat16(), t.bfloat16() if mt else None, w, b, act,
+                                 out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        assert torch.equal(got[0], ref[0])
+        assert not mt or torch.equal(got[1], ref[1])
