@@ -533,8 +533,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         const int steps = ke - kb;
         // steps 0 and 1: group 0 loads A, group 1 B
         issue(0, kb, grp);
-        if (steps > 1) issue(1, kb + 1, grp);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (steps > 1) {
+            issue(1, kb + 1, grp);
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");   // step 0; step 1 as in the loop
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         barrier();
         if (grp == 1) barrier();
 #pragma unroll 1
@@ -1304,13 +1308,18 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             const int hi = owner((long)t * nk + nk - 1);
             if (arrival == hi - lo) {
                 // sum every part, this one's included, in workgroup order so
-                // that the result does not depend on the order of arrival
+                // that the result does not depend on the order of arrival; of
+                // two parts only the other is read (p0 + p1 either way round)
+                const bool two = hi == lo + 1;
+                if (!two) {
 #pragma unroll
-                for (int ii = 0; ii < 8; ++ii)
+                    for (int ii = 0; ii < 8; ++ii)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[ii][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        for (int j = 0; j < 4; ++j) acc[ii][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
 #pragma unroll 1
                 for (int q = lo; q <= hi; ++q) {
+                    if (two && q == s) continue;
                     const __amdgpu_buffer_rsrc_t other = __builtin_amdgcn_make_buffer_rsrc(
                         sk.slots + (long)q * kSlotFloats, (short)0, kSlotFloats * 4, kRawBufferFormat);
                     // sixteen 16-byte loads in flight per batch (sixteen
