@@ -59,6 +59,33 @@ struct LinearResidual {
     const float* gate_s[2];    // the stream's own [n] vector, or null
     AdaRows rows;
 };
+// The VAE attention's products on the 256-tile GEMM (bf16 rows, k % 64 == 0):
+// per-row operands, and a gate: a launch whose *gate is not gate_want ends at
+// once (a null gate always runs).  ref, scale and a row of sums span m
+// rounded up to 256.
+struct LinearRows {
+    const float* ref;     // launch_linear_exp: log2-domain reference of each row
+    float* sums;          // its partial row sums, [2 ceil(n / 256)][sums_pitch]
+    int sums_pitch;
+    int pitch;            // its output row pitch (n <= pitch, multiple of 8)
+    const float* scale;   // launch_linear_row_scale: factor of each row
+    const int* gate;
+    int gate_want;
+    int ld;               // row pitch of both operands, a multiple of 8 (0: k)
+};
+// y[r][c] = exp2(log2(e) (q keys^T)[r][c] - ref[r]) for c < n, 0 for n <= c <
+// pitch, bf16, over m rows of q and n keys; sums[t][r] the fp32 sum of row r's
+// values in columns [128 t, + 128)
+hipError_t launch_linear_exp(const uint16_t* q, int m, const uint16_t* keys, int n, int k,
+                             uint16_t* y, const LinearRows& lr, hipStream_t stream);
+// y = (x W^T) scale[r] + bias, bf16 [m][n], n % 8 == 0
+hipError_t launch_linear_row_scale(const uint16_t* x, int m, const uint16_t* w, const float* bias,
+                                   int n, int k, uint16_t* y, const LinearRows& lr,
+                                   hipStream_t stream);
+// y = x W^T, fp32 [m][n], behind the gate
+hipError_t launch_linear_gated(const uint16_t* x, int m, const uint16_t* w, int n, int k, float* y,
+                               const LinearRows& lr, hipStream_t stream);
+
 // y = x W^T + b over the two streams (bf16 activations, k % 64 == 0,
 // n % 8 == 0) with the residual epilogue in place of the y stores.
 hipError_t launch_shared_linear_residual(const uint16_t* x0, int m0, const uint16_t* x1, int m1,

@@ -99,7 +99,19 @@ MhaWeights mha_layout(const s2_mha_config* c) {
 struct MhaWork {
     int lp;   // seq rounded up to 64: the k extent of the P V product
     size_t xp, q, k, vt, s, p, oh, o, total;
+    // exponentials taken in the score product's epilogue: their scratch
+    bool fused;
+    int pitch, parts;   // rows rounded up to the GEMM's 256; row sums per row
+    size_t stats, ref, sums, scale, general;
 };
+
+// Sequences from here on take the exponentials in the score product's
+// epilogue, one head (whose q and k come from one product), or several.  The
+// small launches around it cost what the fp32 score matrix and its softmax
+// pass cost at some length: one head of 512, bf16, 256 tokens 104 against 102
+// us, 1024 tokens 112 against 122, 14,400 tokens 540 against 810; with q and k
+// apart 3001 tokens 152 against 151, 4096 tokens 159 against 164.
+constexpr int kMhaFusedSeq = 1024, kMhaFusedSeqHeads = 4096;
 
 MhaWork mha_work(const s2_mha_config* c, int seq) {
     MhaWork w;
@@ -114,6 +126,18 @@ MhaWork mha_work(const s2_mha_config* c, int seq) {
     w.oh = w.p + align256((size_t)seq * w.lp * 2);
     w.o = w.oh + align256((size_t)seq * d * 2);
     w.total = w.o + (c->num_heads > 1 ? align256((size_t)seq * c->embed_dim * 2) : 0);
+    w.fused = seq >= (c->num_heads == 1 ? kMhaFusedSeq : kMhaFusedSeqHeads) && d % 64 == 0 && (long)256 * w.lp * 4 <= 0x7fffffffL &&
+              (long)512 * d * 4 <= 0x7fffffffL;
+    if (w.fused) {
+        w.pitch = (seq + 255) / 256 * 256;
+        w.parts = 2 * ((seq + 255) / 256);
+        w.stats = w.total;
+        w.ref = w.stats + align256((size_t)3 * w.pitch * 4);
+        w.sums = w.ref + align256((size_t)w.pitch * 4);
+        w.scale = w.sums + align256((size_t)w.parts * w.pitch * 4);
+        w.general = w.scale + align256((size_t)w.pitch * 4);
+        w.total = w.general + 256;
+    }
     return w;
 }
 
@@ -1506,21 +1530,62 @@ int s2_mha_forward(const s2_mha_config* config, const void* prepared, const void
     hipStream_t st = (hipStream_t)stream;
     constexpr int kBF = (int)S2_DTYPE_BF16, kF32 = (int)S2_DTYPE_F32;
     // x as bf16 rows, padded with zero rows to the 64-multiple extent of P V
-    S2_HIP(s2::launch_mha_stage(x, (int)in_dtype, seq, w.lp, Q, xp, st));
+    // (bf16 rows that need no padding are read in place)
+    if (in_dtype == S2_DTYPE_BF16 && w.lp == seq)
+        xp = (uint16_t*)const_cast<void*>(x);
+    else
+        S2_HIP(s2::launch_mha_stage(x, (int)in_dtype, seq, w.lp, Q, xp, st));
     for (int h = 0; h < H; ++h) {
         const long wo_h = (long)h * D * Q;
-        // q_h = x Wq_h^T + bq_h (scale folded in), k_h likewise: [lp][D]
-        S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wq + wo_h, bq + h * D, D, Q,
-                                        S2_ACT_NONE, q, nullptr, kBF, st));
-        S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wk + wo_h, bk + h * D, D, Q,
-                                        S2_ACT_NONE, k, nullptr, kBF, st));
+        // q_h = x Wq_h^T + bq_h (scale folded in), k_h likewise: [lp][D]; with
+        // one head and no gap between the two weights and biases, one product
+        // makes [lp][q | k]
+        const bool joint = w.fused && m.wk == (size_t)E * Q * 2 && m.bk - m.bq == (size_t)E * 4 && H == 1;
+        const int ld = joint ? 2 * D : D;
+        const uint16_t* kh = joint ? q + D : k;
+        if (joint) {
+            S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wq, bq, 2 * D, Q, S2_ACT_NONE,
+                                            q, nullptr, kBF, st));
+        } else {
+            S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wq + wo_h, bq + h * D, D, Q,
+                                            S2_ACT_NONE, q, nullptr, kBF, st));
+            S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wk + wo_h, bk + h * D, D, Q,
+                                            S2_ACT_NONE, k, nullptr, kBF, st));
+        }
         // v_h^T without its bias = Wv_h x^T: [D][lp], zero columns past seq
         S2_HIP(s2::launch_shared_linear(wv + wo_h, D, nullptr, 0, kBF, xp, nullptr, w.lp, Q,
                                         S2_ACT_NONE, vt, nullptr, kBF, st));
+        if (w.fused) {
+            // P = exp(q_h k_h^T - reference), its row sums, and o_h = P v_h
+            // over them; or the scores and their softmax where `general` says so
+            s2::LinearRows lr = {};
+            lr.ref = (const float*)(ws + w.ref);
+            lr.sums = (float*)(ws + w.sums);
+            lr.sums_pitch = w.pitch;
+            lr.pitch = w.lp;
+            lr.scale = (const float*)(ws + w.scale);
+            int* general = (int*)(ws + w.general);
+            lr.ld = ld;
+            S2_HIP(s2::launch_mha_reference(q, kh, ld, seq, D, w.pitch, (float*)(ws + w.stats),
+                                            (float*)(ws + w.ref), general, st));
+            lr.gate = general;
+            lr.gate_want = 0;
+            S2_HIP(s2::launch_linear_exp(q, seq, kh, seq, D, p, lr, st));
+            lr.gate_want = 1;
+            S2_HIP(s2::launch_linear_gated(q, seq, kh, seq, D, sc, lr, st));
+            S2_HIP(s2::launch_mha_softmax(sc, seq, seq, seq, w.lp, p, general, st));
+            S2_HIP(s2::launch_mha_row_scale(lr.sums, w.parts, w.pitch, general,
+                                            (float*)(ws + w.scale), seq, st));
+            lr.gate = nullptr;
+            lr.ld = 0;
+            S2_HIP(s2::launch_linear_row_scale(p, seq, vt, bv + h * D, D, w.lp, oh, lr, st));
+            if (H > 1) S2_HIP(s2::launch_mha_interleave(oh, seq, D, E, h, o, st));
+            continue;
+        }
         // S = q_h k_h^T (already scaled): [seq][seq] fp32
         S2_HIP(s2::launch_shared_linear(q, seq, nullptr, 0, kBF, k, nullptr, seq, D, S2_ACT_NONE,
                                         sc, nullptr, kF32, st));
-        S2_HIP(s2::launch_mha_softmax(sc, seq, seq, seq, w.lp, p, st));
+        S2_HIP(s2::launch_mha_softmax(sc, seq, seq, seq, w.lp, p, nullptr, st));
         // o_h = P v_h + bv_h (the rows of P sum to one): [seq][D]
         S2_HIP(s2::launch_shared_linear(p, seq, nullptr, 0, kBF, vt, bv + h * D, D, w.lp,
                                         S2_ACT_NONE, oh, nullptr, kBF, st));

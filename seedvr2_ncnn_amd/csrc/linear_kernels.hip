@@ -309,13 +309,22 @@ struct AwaQkvArgs {
     uint16_t* vt;
 };
 
+// Epilogues of the VAE attention's products (one stream, bf16 output):
+//   kActExp       rows are keys, columns queries: y[query][key] = exp(acc -
+//                 reference of the query), zeros for keys past m0 up to the
+//                 row pitch, and per 128 keys the fp32 sums of a query's values.
+//                 A lane holds four consecutive keys of a query: packed
+//                 conversions, 8-byte LDS writes and sums within the lane
+//   kActRowScale  y = acc * (scale of the row) + bias
+constexpr int kActExp = 100, kActRowScale = 101;
+
 // XK is the element type of x0 and x1 (0 fp32, 1 bf16, 2 fp16).
 template <int YK, int ACT, int AWA = 0, int RES = 0, int XK = 1>
 __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     const uint16_t* __restrict__ x0, int m0, const uint16_t* __restrict__ x1, int m1,
     const uint16_t* __restrict__ wgt, const float* __restrict__ bias, int n, int k,
     void* __restrict__ y0, void* __restrict__ y1, int mv, int mtiles, int ntiles, SkTail sk,
-    AwaQkvArgs awa, LinearResidual res) {
+    AwaQkvArgs awa, LinearResidual res, LinearRows lr) {
     constexpr int BM = 256, BN = 256, BK = 64;
     constexpr int TB = BM * BK * 2;   // 32 KB per operand per stage
     constexpr int SB = 2 * TB;        // 64 KB per stage
@@ -330,6 +339,9 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // four A-loading waves, eight per lane (read back at each DMA issue:
     // the main loop has no registers to spare for them)
     __shared__ uint4 goff_lds[AWA ? 4 * 64 * 2 : 1];
+
+    if constexpr (AWA == 0 && RES == 0)
+        if (lr.gate && *lr.gate != lr.gate_want) return;   // uniform: no workgroup waits
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -360,7 +372,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // output row of tile row rl, or null past either stream
     // output row pitch: n, or n / 2 for SwiGLU, whose weight has a gate and
     // an up row per output column
-    const int ny = ACT == S2_ACT_SWIGLU ? n / 2 : n;
+    const int ny = ACT == S2_ACT_SWIGLU ? n / 2 : ACT == kActExp ? lr.pitch : n;
     auto out_row = [&](int rl) -> void* {
         const int r = row0 + rl;
         if (r < m0) return (char*)y0 + (long)r * ny * (YK ? 2 : 4);
@@ -404,7 +416,55 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // 16-bit values in the LDS staging rows (pitch EP); the 16-bit outputs
     // of the plain epilogue
     auto stage_own_rows = [&]() {
-        if constexpr (YK != 0 && AWA == 0 && ACT != S2_ACT_SWIGLU) {
+        if constexpr (ACT == kActExp) {
+            constexpr float kLog2e = 1.4426950408889634f;
+            const EpiIds ei = epi_ids();
+            auto stage = [&](auto full_tag) {
+                constexpr bool FULL = decltype(full_tag)::value;   // no key past m0
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int cl = ei.wn * 64 + 16 * j + ei.l16;
+                    const float ref = lr.ref[col0 + cl];
+                    float sum = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
+                        float v[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            v[r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], kLog2e, -ref));
+                            if (!FULL && row0 + rl + r >= m0) v[r] = 0.f;
+                        }
+                        sum += (v[0] + v[1]) + (v[2] + v[3]);
+                        *(uint2*)(lds + cl * EP + rl * 2) =
+                            make_uint2(pack2_bf16_rne(v[0], v[1]), pack2_bf16_rne(v[2], v[3]));
+                    }
+                    sum += __shfl_xor(sum, 16);
+                    sum += __shfl_xor(sum, 32);
+                    if (ei.g == 0)
+                        lr.sums[(long)(row0 / 128 + ei.wm) * lr.sums_pitch + col0 + cl] = sum;
+                }
+            };
+            if (row0 + BM <= m0)
+                stage(std::true_type{});
+            else
+                stage(std::false_type{});
+        } else if constexpr (ACT == kActRowScale) {
+            const EpiIds ei = epi_ids();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
+                const f32x4 sc = *reinterpret_cast<const f32x4*>(lr.scale + row0 + rl);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int cl = ei.wn * 64 + 16 * j + ei.l16;
+                    const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        *(__bf16*)(lds + (rl + r) * EP + cl * 2) = (__bf16)fmaf(acc[i][j][r], sc[r], bv);
+                }
+            }
+        } else if constexpr (YK != 0 && AWA == 0 && ACT != S2_ACT_SWIGLU) {
             const EpiIds ei = epi_ids();
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -447,24 +507,25 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     auto mainloop = [&](int kb, int ke, bool early) {
         const int grp = wave >> 2;
         const int wq = wave & 3;
+        const int ld = lr.ld ? lr.ld : k;   // row pitch of x and of the weight
         // plain: the tile's rows of each stream; fused QKV: whole streams,
         // each DMA lane addressing its gathered row
         const i32x4 rav = AWA ? wave_uniform(buffer_rsrc(x0, (uint32_t)((long)m0 * k * 2)))
                               : wave_uniform(buffer_rsrc(
-                                    x0 + (long)row0 * k, (uint32_t)(max(min(m0 - row0, BM), 0) * k * 2)));
+                                    x0 + (long)row0 * ld, (uint32_t)(max(min(m0 - row0, BM), 0) * ld * 2)));
         const i32x4 rat =
             AWA ? wave_uniform(buffer_rsrc(x1, (uint32_t)((long)m1 * k * 2)))
-                : wave_uniform(buffer_rsrc(x1 + (long)(row0 - mv) * k,
-                                           (uint32_t)(row0 + BM > mv ? min(mv + m1 - row0, BM) * k * 2 : 0)));
+                : wave_uniform(buffer_rsrc(x1 + (long)(row0 - mv) * ld,
+                                           (uint32_t)(row0 + BM > mv ? min(mv + m1 - row0, BM) * ld * 2 : 0)));
         const int wrow = __builtin_amdgcn_readfirstlane(row0 + wq * 64);
         const i32x4 rb =
-            wave_uniform(buffer_rsrc(wgt + (long)col0 * k, (uint32_t)(min(n - col0, BN) * k * 2)));
+            wave_uniform(buffer_rsrc(wgt + (long)col0 * ld, (uint32_t)(min(n - col0, BN) * ld * 2)));
         // Wave wq of a group fills LDS rows 64 wq .. 64 wq + 63 of its operand
         // (group 0: A, group 1: B) with 8 DMA instructions of 8 rows.  Row
         // r + 8j has the swizzle of row r with bit 2 flipped for odd j, so two
         // offsets serve all eight.
         const int row_a = wq * 64 + (lane >> 3);
-        const uint32_t vrow = (uint32_t)(row_a * k * 2);
+        const uint32_t vrow = (uint32_t)(row_a * ld * 2);
         const uint32_t voff_even = vrow + (((lane & 7) ^ lds_swizzle(row_a)) * 16);
         const uint32_t voff_odd = vrow + (((lane & 7) ^ lds_swizzle(row_a) ^ 4) * 16);
         // fused QKV: byte offsets of this lane's eight gathered A rows (a gap
@@ -499,7 +560,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                uint32_t vo = ((j & 1) ? voff_odd : voff_even) + (uint32_t)(j * 8 * k * 2);
+                uint32_t vo = ((j & 1) ? voff_odd : voff_even) + (uint32_t)(j * 8 * ld * 2);
                 if constexpr (AWA != 0)
                     if (!operand) vo = go[j];
                 lds_dma16(operand ? rb : (wrow + j * 8 < mv ? rav : rat),
@@ -1095,7 +1156,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             return;
         }
         const EpiIds ei = epi_ids();
-        if (YK && (n & 7) == 0) {
+        if (YK && (ny & 7) == 0) {
             if constexpr (RES == 0) {
                 // Thread t of group g (waves 4g .. 4g + 3) stores 16-byte
                 // chunk t%32 of rows 128g + t/32 + 8c, all sixteen LDS reads
@@ -1129,8 +1190,27 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 const int ch = t & 31;
                 const int sub = t >> 5;
                 const int lw = ei.wn;   // wave within the group
-                const uint32_t drop = col0 + ch * 8 < n ? 0u : 0x80000000u;
+                const uint32_t drop = col0 + ch * 8 < ny ? 0u : 0x80000000u;
                 auto store_rows = [&]() {
+                    if constexpr (ACT == kActExp) {
+                        // 16-byte chunk t%16 of this group's 128 keys, queries
+                        // t/16 + 16c
+                        const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+                            (char*)y0 + (long)col0 * pitch, (short)0, min(n - col0, BN) * pitch,
+                            kRawBufferFormat);
+                        const int key = row0 + 128 * g0 + (t & 15) * 8;
+                        const uint32_t past = key < ny ? 0u : 0x80000000u;
+                        u32x4 qv[16];
+#pragma unroll
+                        for (int c = 0; c < 16; ++c)
+                            qv[c] = *(const u32x4*)(lds + ((t >> 4) + 16 * c) * EP + 256 * g0 + (t & 15) * 16);
+#pragma unroll
+                        for (int c = 0; c < 16; ++c)
+                            __builtin_amdgcn_raw_buffer_store_b128(
+                                qv[c], rq, (uint32_t)(((t >> 4) + 16 * c) * pitch + key * 2) | past, 0,
+                                kNonTemporal);
+                        return;
+                    }
                     u32x4 sv[16];
 #pragma unroll
                     for (int c = 0; c < 16; ++c)
@@ -1274,8 +1354,9 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         // the plain 16-bit epilogue of a whole tile without an activation runs
         // early (see epilogue); with GELU the early schedule would serialise
         // the two groups' VALU work, which otherwise shares the SIMDs
-        const bool early = AWA == 0 && RES == 0 && XK == 1 && ACT == S2_ACT_NONE && YK != 0 &&
-                           (n & 7) == 0 && finish;
+        const bool early = AWA == 0 && RES == 0 && XK == 1 &&
+                           (ACT == S2_ACT_NONE || ACT == kActExp || ACT == kActRowScale) &&
+                           YK != 0 && (ny & 7) == 0 && finish;
         if constexpr (XK == 1)
             mainloop(kb, ke, early);
         else
@@ -1558,7 +1639,7 @@ static hipError_t linear_impl(const void* x0, int m0, const void* x1, int m1, co
         const long blocks = (long)sk.dp_tiles + sk.sk_groups;
         shared_linear_256_kernel<YK, ACT, 0, 0, XK><<<(unsigned)blocks, 512, 0, stream>>>(
             (const uint16_t*)x0, m0, (const uint16_t*)x1, m1, w, bias, n, k, y0, y1, mv, mtiles,
-            ntiles, sk, AwaQkvArgs{}, LinearResidual{});
+            ntiles, sk, AwaQkvArgs{}, LinearResidual{}, LinearRows{});
         return hipGetLastError();
     }
     const int mt0 = (m0 + 127) / 128;
@@ -1646,8 +1727,47 @@ hipError_t launch_shared_linear_residual(const uint16_t* x0, int m0, const uint1
     const long blocks = (long)sk.dp_tiles + sk.sk_groups;
     shared_linear_256_kernel<1, S2_ACT_NONE, 0, 1><<<(unsigned)blocks, 512, 0, stream>>>(
         x0, m0, x1, m1, w, bias, n, k, nullptr, nullptr, mv, mtiles, ntiles, sk, AwaQkvArgs{},
-        res);
+        res, LinearRows{});
     return hipGetLastError();
+}
+
+// One stream of bf16 rows on the 256-tile kernel with the epilogue ACT of
+// LinearRows.
+template <int YK, int ACT>
+static hipError_t linear_rows(const uint16_t* x, int m, const uint16_t* w, const float* bias, int n,
+                              int k, void* y, const LinearRows& lr, hipStream_t stream) {
+    const long row = ACT == kActExp ? lr.pitch : n;   // output row pitch
+    if (m <= 0 || n <= 0 || k % 64 != 0 || (YK && row % 8 != 0) || lr.ld % 8 != 0 ||
+        (long)256 * std::max(k, lr.ld) * 2 > 0x7fffffffL ||
+        256 * row * 4 > 0x7fffffffL)
+        return hipErrorInvalidValue;
+    const int mv = (m + 7) / 8 * 8;
+    const int ntiles = (n + 255) / 256;
+    const int mtiles = (mv + 255) / 256;
+    SkTail sk;
+    hipError_t e = plan_sk_tail((long)mtiles * ntiles, k / 64, SkSource::kStream, stream, &sk);
+    if (e != hipSuccess) return e;
+    const long blocks = (long)sk.dp_tiles + sk.sk_groups;
+    shared_linear_256_kernel<YK, ACT><<<(unsigned)blocks, 512, 0, stream>>>(
+        x, m, nullptr, 0, w, bias, n, k, y, nullptr, mv, mtiles, ntiles, sk, AwaQkvArgs{},
+        LinearResidual{}, lr);
+    return hipGetLastError();
+}
+
+hipError_t launch_linear_exp(const uint16_t* q, int m, const uint16_t* keys, int n, int k,
+                             uint16_t* y, const LinearRows& lr, hipStream_t stream) {
+    return linear_rows<1, kActExp>(keys, n, q, nullptr, m, k, y, lr, stream);
+}
+
+hipError_t launch_linear_row_scale(const uint16_t* x, int m, const uint16_t* w, const float* bias,
+                                   int n, int k, uint16_t* y, const LinearRows& lr,
+                                   hipStream_t stream) {
+    return linear_rows<1, kActRowScale>(x, m, w, bias, n, k, y, lr, stream);
+}
+
+hipError_t launch_linear_gated(const uint16_t* x, int m, const uint16_t* w, int n, int k, float* y,
+                               const LinearRows& lr, hipStream_t stream) {
+    return linear_rows<0, S2_ACT_NONE>(x, m, w, nullptr, n, k, y, lr, stream);
 }
 
 hipError_t launch_awa_qkv(const s2_awa_plan& plan, const uint16_t* x_video, const uint16_t* x_text,
@@ -1685,11 +1805,11 @@ hipError_t launch_awa_qkv(const s2_awa_plan& plan, const uint16_t* x_video, cons
     if (d == 128)
         shared_linear_256_kernel<1, S2_ACT_NONE, 128><<<(unsigned)blocks, 512, 0, stream>>>(
             x_video, plan.video_tokens, x_text, plan.text_tokens, w, bias, n, k, nullptr, nullptr,
-            plan.qkv_text_row, mtiles, ntiles, sk, a, LinearResidual{});
+            plan.qkv_text_row, mtiles, ntiles, sk, a, LinearResidual{}, LinearRows{});
     else
         shared_linear_256_kernel<1, S2_ACT_NONE, 64><<<(unsigned)blocks, 512, 0, stream>>>(
             x_video, plan.video_tokens, x_text, plan.text_tokens, w, bias, n, k, nullptr, nullptr,
-            plan.qkv_text_row, mtiles, ntiles, sk, a, LinearResidual{});
+            plan.qkv_text_row, mtiles, ntiles, sk, a, LinearResidual{}, LinearRows{});
     return hipGetLastError();
 }
 

@@ -7,9 +7,11 @@
 // few query rows per wave (a 16-row x 512 fp32 output tile is 128 registers
 // per lane) and its K/V fragment reads from LDS outgrow the matrix-core
 // time.  With 288 GB of HBM the score matrix fits many times over, so the
-// forward runs through the SharedLinear GEMM instead: the projections, S =
-// Q K^T in fp32, a row softmax into bf16 P, O = P V, and the output
-// projection.  This file holds the kernels between the GEMMs.
+// forward runs through the SharedLinear GEMM instead: the projections, P =
+// exp(Q K^T - reference) in bf16 with the fp32 row sums from the same epilogue,
+// O = P V scaled by them, and the output projection.  Short sequences, and
+// heads whose scores no reference covers, take S = Q K^T in fp32 and a row
+// softmax into bf16 P instead.  This file holds the kernels between the GEMMs.
 #include <math.h>
 
 #include "mha_kernels.h"
@@ -18,26 +20,141 @@
 namespace s2 {
 namespace {
 
-// rows [0, rows) of x (element type `kind`, row stride qdim) -> bf16 rows of
-// xp [rows_padded][qdim]; rows at or above `rows` are zero
+// the first `valid` of `total` elements of x (element type KIND), as bf16,
+// and zeros for the rest; both are multiples of 8, which a thread moves
+// (one element a thread took 19 us for 14400 rows of 512)
 template <int KIND>
-__global__ __launch_bounds__(256) void mha_stage_kernel(const void* __restrict__ x, int rows,
-                                                        int rows_padded, int qdim,
-                                                        uint16_t* __restrict__ xp) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    const long total = (long)rows_padded * qdim;
+__global__ __launch_bounds__(256) void mha_stage_kernel(const void* __restrict__ x, long valid,
+                                                        long total, uint16_t* __restrict__ xp) {
+    const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
     if (i >= total) return;
-    const long r = i / qdim;
-    float v = 0.f;
-    if (r < rows) {
-        if (KIND == 1)
-            v = __builtin_bit_cast(float, (uint32_t)((const uint16_t*)x)[i] << 16);
-        else if (KIND == 2)
-            v = (float)((const _Float16*)x)[i];
-        else
-            v = ((const float*)x)[i];
+    uint4 out = make_uint4(0u, 0u, 0u, 0u);
+    if (i < valid) {
+        if (KIND == 1) {
+            out = *reinterpret_cast<const uint4*>((const uint16_t*)x + i);
+        } else {
+            float v[8];
+            if (KIND == 2) {
+                const uint4 u = *reinterpret_cast<const uint4*>((const uint16_t*)x + i);
+                const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    v[e] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+            } else {
+                load8((const float*)x + i, v);
+            }
+            out = cvt8_bf16(v);
+        }
     }
-    xp[i] = f32_to_bf16(v);
+    *reinterpret_cast<uint4*>(xp + i) = out;
+}
+
+// ---- the exponentials' reference -------------------------------------------
+//
+// The scores of row r are bounded by B_r = |q_r| max_j |k_j| (log2 domain,
+// with 2^-6 of slack for the products' rounding).  Their exponentials are
+// taken relative to c_r = max(0, B_r - 80): no value exceeds 2^80, so the sums
+// of a row and of its product with V stay finite, and as long as the row's
+// largest score lies within 180 of B_r its probabilities stay above 2^-100,
+// with 2^-26 of them still normal numbers.  A row's own key shows that: the
+// reference is good for a head when q_r k_r >= B_r - 180 for every row.
+// Otherwise (also for non-finite operands) `general` sends the head through
+// fp32 scores and the softmax pass.
+
+// |q_r|^2, |k_r|^2 and q_r k_r, one wave a row (row pitch ld); clears the flag
+__global__ __launch_bounds__(256) void mha_norms_kernel(const uint16_t* __restrict__ q,
+                                                        const uint16_t* __restrict__ k, int ld,
+                                                        int rows, int d, int pitch,
+                                                        float* __restrict__ stats,
+                                                        int* __restrict__ general) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *general = 0;
+    const int r = (int)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (r >= rows) return;
+    float qq = 0.f, kk = 0.f, qk = 0.f;
+    for (int c = lane * 8; c < d; c += 512) {
+        float a[8], b[8];
+        load8(q + (long)r * ld + c, a);
+        load8(k + (long)r * ld + c, b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            qq = fmaf(a[e], a[e], qq);
+            kk = fmaf(b[e], b[e], kk);
+            qk = fmaf(a[e], b[e], qk);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        qq += __shfl_xor(qq, off);
+        kk += __shfl_xor(kk, off);
+        qk += __shfl_xor(qk, off);
+    }
+    if (lane == 0) {
+        stats[r] = qq;
+        stats[pitch + r] = kk;
+        stats[2 * pitch + r] = qk;
+    }
+}
+
+// c_r of every row (0 in the padding up to `pitch`) and the head's `general`
+// flag: a block takes 256 rows, and finds the largest |k_j| itself (one block
+// for all rows took 12-14 us for 14,400 of them)
+__global__ __launch_bounds__(256) void mha_reference_kernel(const float* __restrict__ stats,
+                                                            int rows, int pitch,
+                                                            float* __restrict__ ref,
+                                                            int* __restrict__ general) {
+    constexpr float kLog2e = 1.4426950408889634f;
+    __shared__ float red[4];
+    const int t = threadIdx.x;
+    const int r = blockIdx.x * 256 + t;
+    // (statistics past `rows` are read and not used; pitch % 256 == 0)
+    const float qq = stats[r], own = stats[2 * pitch + r] * kLog2e;
+    float m = 0.f;
+    int bad = 0;
+#pragma unroll 8
+    for (int i = t * 4; i < rows; i += 1024) {
+        const float4 kk = *reinterpret_cast<const float4*>(stats + pitch + i);
+        const float v[4] = {kk.x, kk.y, kk.z, kk.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (i + e >= rows) continue;
+            bad |= !(v[e] <= 3.0e38f);   // also for NaN
+            m = fmaxf(m, v[e]);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if ((t & 63) == 0) red[t >> 6] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    const float b = sqrtf(qq) * sqrtf(m) * (kLog2e * (1.f + 0.015625f));
+    const bool in = r < rows;
+    bad |= in && !(own >= b - 180.f);
+    ref[r] = in ? fmaxf(b - 80.f, 0.f) : 0.f;
+    if (__any(bad) && (t & 63) == 0)
+        __hip_atomic_store(general, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// 1 / (sum of a row's exponentials over the column parts), or 1 when the
+// probabilities are already normalised; a block takes 64 rows, its waves
+// every fourth part
+__global__ __launch_bounds__(256) void mha_row_scale_kernel(const float* __restrict__ sums, int parts,
+                                                            int pitch, const int* __restrict__ general,
+                                                            float* __restrict__ scale, int rows) {
+    __shared__ float red[4][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = blockIdx.x * 64 + l;   // pitch is a multiple of 64
+    float s = 0.f;
+    if (!*general) {
+#pragma unroll 8
+        for (int i = w; i < parts; i += 4) s += sums[(long)i * pitch + r];
+    }
+    red[w][l] = s;
+    __syncthreads();
+    if (w == 0) {
+        s = (red[0][l] + red[1][l]) + (red[2][l] + red[3][l]);
+        scale[r] = r < rows && !*general ? 1.f / s : 1.f;
+    }
 }
 
 // weights: fp32 -> bf16, times `scale`
@@ -59,8 +176,10 @@ __global__ __launch_bounds__(256) void mha_bias_kernel(const float* __restrict__
 // L2, to write P.
 __global__ __launch_bounds__(256) void mha_softmax_kernel(const float* __restrict__ s, long ld_s,
                                                           int cols, int ld_p,
-                                                          uint16_t* __restrict__ p) {
+                                                          uint16_t* __restrict__ p,
+                                                          const int* __restrict__ gate) {
     constexpr float kLog2e = 1.4426950408889634f;
+    if (gate && !*gate) return;
     __shared__ float red_m[4], red_s[4];
     const float* row = s + (long)blockIdx.x * ld_s;
     uint16_t* out = p + (long)blockIdx.x * ld_p;
@@ -107,8 +226,10 @@ __global__ __launch_bounds__(256) void mha_softmax_kernel(const float* __restric
 template <int NV, bool VEC>
 __global__ __launch_bounds__(256) void mha_softmax_reg_kernel(const float* __restrict__ s,
                                                               long ld_s, int cols, int ld_p,
-                                                              uint16_t* __restrict__ p) {
+                                                              uint16_t* __restrict__ p,
+                                                              const int* __restrict__ gate) {
     constexpr float kLog2e = 1.4426950408889634f;
+    if (gate && !*gate) return;
     __shared__ float red[4];
     const float* row = s + (long)blockIdx.x * ld_s;
     uint16_t* out = p + (long)blockIdx.x * ld_p;
@@ -176,14 +297,30 @@ unsigned blocks(long n) { return (unsigned)((n + 255) / 256); }
 
 hipError_t launch_mha_stage(const void* x, int kind, int rows, int rows_padded, int qdim,
                             uint16_t* xp, hipStream_t stream) {
-    const long total = (long)rows_padded * qdim;
+    const long valid = (long)rows * qdim, total = (long)rows_padded * qdim;   // qdim % 8 == 0
     if (total <= 0) return hipSuccess;
     if (kind == 1)
-        mha_stage_kernel<1><<<blocks(total), 256, 0, stream>>>(x, rows, rows_padded, qdim, xp);
+        mha_stage_kernel<1><<<blocks(total / 8), 256, 0, stream>>>(x, valid, total, xp);
     else if (kind == 2)
-        mha_stage_kernel<2><<<blocks(total), 256, 0, stream>>>(x, rows, rows_padded, qdim, xp);
+        mha_stage_kernel<2><<<blocks(total / 8), 256, 0, stream>>>(x, valid, total, xp);
     else
-        mha_stage_kernel<0><<<blocks(total), 256, 0, stream>>>(x, rows, rows_padded, qdim, xp);
+        mha_stage_kernel<0><<<blocks(total / 8), 256, 0, stream>>>(x, valid, total, xp);
+    return hipGetLastError();
+}
+
+hipError_t launch_mha_reference(const uint16_t* q, const uint16_t* k, int ld, int rows, int d,
+                                int pitch, float* stats, float* ref, int* general,
+                                hipStream_t stream) {
+    mha_norms_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, stream>>>(q, k, ld, rows, d, pitch, stats,
+                                                                     general);
+    mha_reference_kernel<<<(unsigned)(pitch / 256), 256, 0, stream>>>(stats, rows, pitch, ref, general);
+    return hipGetLastError();
+}
+
+hipError_t launch_mha_row_scale(const float* sums, int parts, int pitch, const int* general,
+                                float* scale, int rows, hipStream_t stream) {
+    mha_row_scale_kernel<<<(unsigned)(pitch / 64), 256, 0, stream>>>(sums, parts, pitch, general,
+                                                                     scale, rows);
     return hipGetLastError();
 }
 
@@ -202,29 +339,31 @@ hipError_t launch_mha_bias(const float* b, int n, float scale, float* out, hipSt
 
 template <int NV>
 static void softmax_reg(const float* s, long ld_s, int rows, int cols, int ld_p, uint16_t* p,
-                        hipStream_t stream) {
+                        const int* gate, hipStream_t stream) {
     if (ld_s % 4 == 0 && ((uintptr_t)s % 16) == 0)
-        mha_softmax_reg_kernel<NV, true><<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p);
+        mha_softmax_reg_kernel<NV, true>
+            <<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p, gate);
     else
-        mha_softmax_reg_kernel<NV, false><<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p);
+        mha_softmax_reg_kernel<NV, false>
+            <<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p, gate);
 }
 
 hipError_t launch_mha_softmax(const float* s, long ld_s, int rows, int cols, int ld_p,
-                              uint16_t* p, hipStream_t stream) {
+                              uint16_t* p, const int* gate, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
     // rows of up to 16,384 columns live in registers (up to 64 floats per
     // thread); longer rows take the streaming kernel
     const int groups = (ld_p + 1023) / 1024;   // float4 groups per thread
     if (ld_p % 4 != 0 || groups > 16)
-        mha_softmax_kernel<<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p);
+        mha_softmax_kernel<<<(unsigned)rows, 256, 0, stream>>>(s, ld_s, cols, ld_p, p, gate);
     else if (groups <= 2)
-        softmax_reg<2>(s, ld_s, rows, cols, ld_p, p, stream);
+        softmax_reg<2>(s, ld_s, rows, cols, ld_p, p, gate, stream);
     else if (groups <= 4)
-        softmax_reg<4>(s, ld_s, rows, cols, ld_p, p, stream);
+        softmax_reg<4>(s, ld_s, rows, cols, ld_p, p, gate, stream);
     else if (groups <= 8)
-        softmax_reg<8>(s, ld_s, rows, cols, ld_p, p, stream);
+        softmax_reg<8>(s, ld_s, rows, cols, ld_p, p, gate, stream);
     else
-        softmax_reg<16>(s, ld_s, rows, cols, ld_p, p, stream);
+        softmax_reg<16>(s, ld_s, rows, cols, ld_p, p, gate, stream);
     return hipGetLastError();
 }
 

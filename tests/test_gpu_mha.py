@@ -90,6 +90,42 @@ def test_mha_vae_frame_rows():
     assert_close(got[rows], ref)
 
 
+# ---- exponentials in the score product's epilogue (long sequences) --------------
+
+def _reference_weights(g, kind, heads):
+    """64 channels a head.  plain: scores near zero.  shifted: q and k share a
+    constant channel of 40, so every score is near 200 and the exponentials
+    need a reference.  general: q's constant channel is another than k's, so
+    the scores are near zero but far below |q| |k| and no reference shows it."""
+    e = 64 * heads
+    ws = _weights(g, e, e)
+    if kind != "plain":
+        for h in range(heads):
+            for i, c in ((0, 0), (2, 0 if kind == "shifted" else 1)):
+                for ch in (0, 1):
+                    ws[i][64 * h + ch] = 0
+                    ws[i + 1][64 * h + ch] = 40 if ch == c else 0
+    return ws
+
+
+@pytest.mark.parametrize("seq,heads", [(1024, 1), (1601, 1), (4096, 2), (4609, 2)])
+@pytest.mark.parametrize("kind", ["plain", "shifted", "general"])
+def test_mha_long_sequences(seq, heads, kind):
+    g = np.random.default_rng(seq + heads)
+    x = g.standard_normal((seq, 64 * heads)).astype(np.float32)
+    ws = _reference_weights(g, kind, heads)
+    got = _run(_device(heads, ws), x)
+    rows = np.concatenate([np.arange(3), g.integers(0, seq, 24), np.arange(seq - 3, seq)]).astype(np.int32)
+    assert_close(got[rows], oracle.mha(x, heads, *ws, rows=rows, threads=16, fast=True))
+
+
+def test_mha_long_sequence_nan_reaches_every_row():
+    g = np.random.default_rng(3)
+    x = g.standard_normal((4700, 64)).astype(np.float32)
+    x[4321, 7] = np.nan
+    assert np.isnan(_run(_device(1, _weights(g, 64, 64)), x)).all()
+
+
 # ---- the ncnn-surface layer (vae_chunked_mha.h:12-50) --------------------------
 
 FP16_TAG = np.frombuffer(np.uint32(0x01306B47).tobytes(), np.float32)
