@@ -197,13 +197,16 @@ def device_count() -> int:
 
 
 def _stream(stream=None):
+    """Handle of `stream`, or of the current device's current stream (read
+    without building a torch Stream, which costs more than a launch's checks)."""
+    if stream is not None:
+        return stream.cuda_stream
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _ints(values):
@@ -303,15 +306,18 @@ class AwaPlan:
         self.close()
 
 
+_DTYPE_CODES = {}
+
+
 def _dtype_code(t):
-    import torch
-    if t.dtype == torch.bfloat16:
-        return DTYPE_BF16
-    if t.dtype == torch.float16:
-        return DTYPE_F16
-    if t.dtype == torch.float32:
-        return DTYPE_F32
-    raise TypeError(f"unsupported dtype {t.dtype}")
+    if not _DTYPE_CODES:
+        import torch
+        _DTYPE_CODES.update({torch.float32: DTYPE_F32, torch.bfloat16: DTYPE_BF16,
+                             torch.float16: DTYPE_F16})
+    code = _DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}")
+    return code
 
 
 def awa_forward(plan: AwaPlan, norm_weights, rope_freqs, video_q, video_k, video_v, text_q,
@@ -322,15 +328,17 @@ def awa_forward(plan: AwaPlan, norm_weights, rope_freqs, video_q, video_k, video
     [L, 3*inner] tensor are fine).  Returns (out_video, out_text)."""
     import torch
     inner = plan.config.heads * plan.config.head_dim
-    ins = (video_q, video_k, video_v, text_q, text_k, text_v)
-    for t in ins:
-        assert t.is_cuda and t.dim() == 2 and t.stride(1) == 1 and t.shape[1] == inner
+    dtype = video_q.dtype
     dt = _dtype_code(video_q)
-    assert all(_dtype_code(t) == dt for t in ins)
-    vs, ts = video_q.stride(0), text_q.stride(0)
-    assert video_k.stride(0) == vs and video_v.stride(0) == vs
-    assert text_k.stride(0) == ts and text_v.stride(0) == ts
-    odt = out_dtype or video_q.dtype
+    strides = []
+    for t in (video_q, video_k, video_v, text_q, text_k, text_v):
+        st = t.stride()
+        assert len(st) == 2 and st[1] == 1 and t.shape[1] == inner and t.is_cuda
+        assert t.dtype == dtype
+        strides.append(st[0])
+    vs, _, _, ts, _, _ = strides
+    assert strides == [vs, vs, vs, ts, ts, ts]
+    odt = out_dtype or dtype
     dev = video_q.device
     if out_video is None:
         out_video = torch.empty((plan.info.video_tokens, inner), dtype=odt, device=dev)
