@@ -314,6 +314,18 @@ struct AwaQkvArgs {
     uint16_t* vt;
 };
 
+// four values of one column, rows `pitch` bytes apart, as 16-bit LDS elements:
+// two pair conversions (one per value otherwise) and four 2-byte writes
+template <int YK>
+__device__ __forceinline__ void stage_rows4(uint8_t* p, int pitch, const float (&v)[4]) {
+    const uint32_t a = YK == 2 ? pack2_f16_rne(v[0], v[1]) : pack2_bf16_rne(v[0], v[1]);
+    const uint32_t b = YK == 2 ? pack2_f16_rne(v[2], v[3]) : pack2_bf16_rne(v[2], v[3]);
+    *(uint16_t*)p = (uint16_t)a;
+    *(uint16_t*)(p + pitch) = (uint16_t)(a >> 16);
+    *(uint16_t*)(p + 2 * pitch) = (uint16_t)b;
+    *(uint16_t*)(p + 3 * pitch) = (uint16_t)(b >> 16);
+}
+
 // Epilogues of the VAE attention's products (one stream, bf16 output):
 //   kActExp       rows are keys, columns queries: y[query][key] = exp(acc -
 //                 reference of the query), zeros for keys past m0 up to the
@@ -464,9 +476,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 for (int j = 0; j < 4; ++j) {
                     const int cl = ei.wn * 64 + 16 * j + ei.l16;
                     const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
+                    float v[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        *(__bf16*)(lds + (rl + r) * EP + cl * 2) = (__bf16)fmaf(acc[i][j][r], sc[r], bv);
+                    for (int r = 0; r < 4; ++r) v[r] = fmaf(acc[i][j][r], sc[r], bv);
+                    stage_rows4<1>(lds + rl * EP + cl * 2, EP, v);
                 }
             }
         } else if constexpr (YK != 0 && AWA == 0 && ACT != S2_ACT_SWIGLU) {
@@ -476,17 +489,16 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 const int cl = ei.wn * 64 + 16 * j + ei.l16;
                 const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
+                for (int i = 0; i < 8; ++i) {
+                    const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
+                    float v[4];
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        float v = acc[i][j][r] + bv;
-                        if (ACT == S2_ACT_GELU) v = gelu(v);
-                        const int rl = ei.wm * 128 + 16 * i + 4 * ei.g + r;
-                        if (YK == 2)
-                            *(_Float16*)(lds + rl * EP + cl * 2) = f32_to_f16(v);
-                        else
-                            *(__bf16*)(lds + rl * EP + cl * 2) = (__bf16)v;
+                        v[r] = acc[i][j][r] + bv;
+                        if (ACT == S2_ACT_GELU) v[r] = gelu(v[r]);
                     }
+                    stage_rows4<YK>(lds + rl * EP + cl * 2, EP, v);
+                }
             }
         }
     };
@@ -833,27 +845,33 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             const int part = col0 / awa.inner;   // 0 q, 1 k, 2 v
             const int hbase = (col0 - part * awa.inner) / D;
             __syncthreads();   // every wave is done reading the last stage
+            auto stage = [&](auto v_tag) {
+                constexpr bool V = decltype(v_tag)::value;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                const float bv = bias ? bias[col0 + cl] : 0.f;
+                for (int j = 0; j < 4; ++j) {
+                    const int cl = ei.wn * 64 + 16 * j + ei.l16;
+                    const float bv = bias ? bias[col0 + cl] : 0.f;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    // the four registers: rows rl .. rl + 3 of column cl
-                    const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
-                    uint16_t hv[4];
+                    for (int i = 0; i < 8; ++i) {
+                        // the four registers: rows rl .. rl + 3 of column cl
+                        const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
+                        float v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        hv[e] = __builtin_bit_cast(uint16_t, (__bf16)(acc[i][j][e] + bv));
-                    if (part < 2) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) *(uint16_t*)(lds + (rl + e) * SP + cl * 2) = hv[e];
-                    } else {
-                        *(uint2*)(lds + cl * SPV + rl * 2) =
-                            make_uint2(hv[0] | ((uint32_t)hv[1] << 16), hv[2] | ((uint32_t)hv[3] << 16));
+                        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bv;
+                        if constexpr (V)
+                            *(uint2*)(lds + cl * SPV + rl * 2) =
+                                make_uint2(pack2_bf16_rne(v[0], v[1]), pack2_bf16_rne(v[2], v[3]));
+                        else
+                            stage_rows4<1>(lds + rl * SP + cl * 2, SP, v);
                     }
                 }
-            }
+            };
+            // one branch for the whole tile: with the choice inside the loop
+            // the compiler branched for every fragment
+            if (part < 2)
+                stage(std::false_type{});
+            else
+                stage(std::true_type{});
             __syncthreads();
             if (part < 2) {
                 constexpr int TPR = D / 8;        // threads per (row, head)
@@ -912,9 +930,13 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 // Only the tile holding the first text row (the row space is
                 // the video rows in window order, then the text rows) selects
                 // between the video and text weights per row.
-                auto passes = [&](auto text_tag) {
+                // (and the rounding mode is one branch around the passes: a
+                // branch in each would keep the compiler from overlapping them)
+                auto passes = [&](auto text_tag, auto official_tag) {
                 constexpr bool TEXT = decltype(text_tag)::value;
+                constexpr bool OFFICIAL = decltype(official_tag)::value;
                 QkvRow ri_next = qrows[etid >> 5];
+                uint4 raw_next = *(const uint4*)(lds + (etid >> 5) * SP + ch * 16);
                 float2 cs_next[4];
                 rope_load(ri_next, cs_next);
 #pragma unroll
@@ -924,12 +946,13 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                     float2 cs[4];
 #pragma unroll
                     for (int pp = 0; pp < 4; ++pp) cs[pp] = cs_next[pp];
+                    const uint4 raw = raw_next;
                     if (pass + 1 < PASSES) {
                         ri_next = qrows[rl + 16];
+                        raw_next = *(const uint4*)(lds + (rl + 16) * SP + ch * 16);
                         rope_load(ri_next, cs_next);
                     }
                     const int kind = ri.pos2 >> 16;
-                    const uint4 raw = *(const uint4*)(lds + rl * SP + ch * 16);
                     const uint32_t wd[4] = {raw.x, raw.y, raw.z, raw.w};
                     float x[8];
 #pragma unroll
@@ -953,7 +976,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                             x[2 * pp + 1] = fmaf(a0, cs[pp].y, a1 * cs[pp].x);
                         }
                     }
-                    if (awa.official_bf16) {
+                    if constexpr (OFFICIAL) {
                         uint16_t hb[8];
 #pragma unroll
                         for (int i = 0; i < 8; ++i) hb[i] = round_bf16_ref_bits(x[i]);
@@ -963,10 +986,13 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                     }
                 }
                 };
-                if (row0 + BM > mv)
-                    passes(std::true_type{});
+                const bool text = row0 + BM > mv;
+                if (awa.official_bf16)
+                    text ? passes(std::true_type{}, std::true_type{})
+                         : passes(std::false_type{}, std::true_type{});
                 else
-                    passes(std::false_type{});
+                    text ? passes(std::true_type{}, std::false_type{})
+                         : passes(std::false_type{}, std::false_type{});
 #pragma unroll
                 for (int pass = 0; pass < PASSES; ++pass) {
                     const QkvRow ri = qrows[pass * 16 + (etid >> 5)];
