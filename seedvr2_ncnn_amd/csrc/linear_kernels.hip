@@ -542,7 +542,8 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         // r + 8j has the swizzle of row r with bit 2 flipped for odd j, so two
         // offsets serve all eight.
         const int row_a = wq * 64 + (lane >> 3);
-        const uint32_t vrow = (uint32_t)(row_a * ld * 2);
+        const uint32_t vrow =
+            (uint32_t)((ACT == S2_ACT_SWIGLU && grp ? wq * 32 + (lane >> 3) : row_a) * ld * 2);
         const uint32_t voff_even = vrow + (((lane & 7) ^ lds_swizzle(row_a)) * 16);
         const uint32_t voff_odd = vrow + (((lane & 7) ^ lds_swizzle(row_a) ^ 4) * 16);
         // fused QKV: byte offsets of this lane's eight gathered A rows (a gap
@@ -578,10 +579,20 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 uint32_t vo = ((j & 1) ? voff_odd : voff_even) + (uint32_t)(j * 8 * ld * 2);
+                uint32_t so = soff;
+                if constexpr (ACT == S2_ACT_SWIGLU)
+                    if (operand) {
+                        // LDS rows 64 wq + 16 q + c of the weight hold gate row
+                        // 32 wq + 16 (q / 2) + c for even q and its up row for
+                        // odd q; no tile of the weight is ragged
+                        const int rj = ((j >> 1) & 1) * 128 + (j >> 2) * 16 + (j & 1) * 8;
+                        vo = (j & 1) ? voff_odd : voff_even;
+                        so = __builtin_amdgcn_readfirstlane(soff + (uint32_t)(rj * ld * 2));
+                    }
                 if constexpr (AWA != 0)
                     if (!operand) vo = go[j];
                 lds_dma16(operand ? rb : (wrow + j * 8 < mv ? rav : rat),
-                          __builtin_amdgcn_readfirstlane(st + j * 1024), vo, soff);
+                          __builtin_amdgcn_readfirstlane(st + j * 1024), vo, so);
             }
         };
         bf16x8 fa[2][8], fb[2][4];
@@ -1019,67 +1030,56 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     };
 
     // SwiGLU: the weight's rows come in blocks of 256, the first 128 gate
-    // rows and the next 128 up rows of the same 128 output columns, so a
-    // tile's columns 0-127 are gates and 128-255 ups of output columns
-    // col0/2 .. col0/2 + 127.  acc + bias is staged as fp32 in two halves of
-    // 128 rows; each thread then forms silu(g) * u for 4 columns of a row.
+    // rows and the next 128 up rows of output columns col0/2 .. col0/2 + 127.
+    // The DMA puts a column's gate and up rows 16 LDS rows apart (issue), so
+    // that a lane's accumulators [i][2q] and [i][2q + 1] are the gate and the
+    // up of column 32 wn + 16 q + l16: silu(g) * u is formed in registers and
+    // staged once, in the output type.  (2464 rows of the v3 MLP: 147 us, 151
+    // with fp32 gates and ups staged in two halves of 128 rows.)
     auto swiglu_epilogue = [&]() {
         if constexpr (ACT == S2_ACT_SWIGLU) {
             const EpiIds ei = epi_ids();
-            constexpr int EF = BN * 4 + 16;   // fp32 row pitch (bytes)
-            const int oc0 = col0 / 2;
+            constexpr int ES = YK ? 2 : 4;
+            constexpr int SP = 128 * ES + 16;   // staged row pitch (bytes)
+            static_assert(BM * SP <= LDS_BYTES, "staged tile exceeds the LDS");
+            __syncthreads();   // every wave is done reading the last stage
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                __syncthreads();   // the stage (h = 0) or the previous half is no longer read
-                if (ei.wm == h) {
+            for (int q = 0; q < 2; ++q) {
+                const int cl = ei.wn * 32 + 16 * q + ei.l16;
+                const bool in = col0 + cl < n;   // n is a multiple of 256
+                const float bg = bias && in ? bias[col0 + cl] : 0.f;
+                const float bu = bias && in ? bias[col0 + 128 + cl] : 0.f;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                        const float bv = bias ? bias[col0 + cl] : 0.f;
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const int rl = 16 * i + 4 * ei.g + r;
-                                *(float*)(lds + rl * EF + cl * 4) = acc[i][j][r] + bv;
-                            }
-                    }
-                }
-                __syncthreads();
-#pragma unroll 2
-                for (int it = 0; it < 8; ++it) {
-                    const int idx = it * 512 + ei.tid;
-                    const int rl = idx >> 5;
-                    const int c4 = (idx & 31) * 4;
-                    const f32x4 gv = *(const f32x4*)(lds + rl * EF + c4 * 4);
-                    const f32x4 uv = *(const f32x4*)(lds + rl * EF + (c4 + 128) * 4);
+                for (int i = 0; i < 8; ++i) {
+                    const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
                     float o[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         // silu(g) = g / (1 + e^-g), e^-g = 2^(-g log2 e)
-                        const float gg = gv[e];
+                        const float gg = acc[i][2 * q][e] + bg;
                         const float sig = __builtin_amdgcn_rcpf(
                             1.f + __builtin_amdgcn_exp2f(-gg * 1.4426950408889634f));
-                        o[e] = gg * sig * uv[e];
+                        o[e] = gg * sig * (acc[i][2 * q + 1][e] + bu);
                     }
-                    void* yr = out_row(h * 128 + rl);
-                    const int col = oc0 + c4;
-                    if (!yr || col >= ny) continue;
-                    if (YK == 0) {
-                        const f32x4 ov = {o[0], o[1], o[2], o[3]};
-                        __builtin_nontemporal_store(ov, (f32x4*)((float*)yr + col));
-                    } else {
-                        uint16_t hb[4];
+                    if constexpr (YK == 0) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            hb[e] = YK == 2 ? __builtin_bit_cast(uint16_t, f32_to_f16(o[e]))
-                                            : __builtin_bit_cast(uint16_t, (__bf16)o[e]);
-                        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-                        const u32x2 hv = {hb[0] | ((uint32_t)hb[1] << 16),
-                                          hb[2] | ((uint32_t)hb[3] << 16)};
-                        __builtin_nontemporal_store(hv, (u32x2*)((uint16_t*)yr + col));
+                        for (int e = 0; e < 4; ++e) *(float*)(lds + (rl + e) * SP + cl * 4) = o[e];
+                    } else {
+                        stage_rows4<YK>(lds + rl * SP + cl * 2, SP, o);
                     }
                 }
+            }
+            __syncthreads();
+            constexpr int CPR = 128 * ES / 16;   // 16-byte chunks per row
+#pragma unroll 8
+            for (int it = 0; it < BM * CPR / 512; ++it) {
+                const int idx = it * 512 + ei.tid;
+                const int rl = idx / CPR, ch = idx % CPR;
+                char* yr = (char*)out_row(rl);
+                const int col = col0 / 2 + ch * (16 / ES);
+                if (yr && col < ny)
+                    __builtin_nontemporal_store(*(const u32x4*)(lds + rl * SP + ch * 16),
+                                                (u32x4*)(yr + (long)col * ES));
             }
         }
     };
