@@ -269,6 +269,7 @@ __device__ __forceinline__ float row_sum(float x) {
 }
 
 constexpr int kSlotFloats = 128 * 512;   // one workgroup's accumulators
+constexpr int kWaveStage = 2 * 32 * 144; // a wave's own LDS in wave_epilogue (bytes)
 
 // Cache policy of the slot stores and loads: sc0 sc1, coherent across the
 // XCDs' L2s (stores write through, loads do not hit a stale L2 line), so the
@@ -429,60 +430,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         return e;
     };
 
-    // acc + bias (and the activation) of this wave's rows of the tile, as
-    // 16-bit values in the LDS staging rows (pitch EP); the 16-bit outputs
-    // of the plain epilogue
+    // acc + bias of this wave's rows of the tile as bf16 values in the LDS
+    // staging rows (pitch EP) of the residual epilogue
     auto stage_own_rows = [&]() {
-        if constexpr (ACT == kActExp) {
-            constexpr float kLog2e = 1.4426950408889634f;
-            const EpiIds ei = epi_ids();
-            auto stage = [&](auto full_tag) {
-                constexpr bool FULL = decltype(full_tag)::value;   // no key past m0
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                    const float ref = lr.ref[col0 + cl];
-                    float sum = 0.f;
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
-                        float v[4];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            v[r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], kLog2e, -ref));
-                            if (!FULL && row0 + rl + r >= m0) v[r] = 0.f;
-                        }
-                        sum += (v[0] + v[1]) + (v[2] + v[3]);
-                        *(uint2*)(lds + cl * EP + rl * 2) =
-                            make_uint2(pack2_bf16_rne(v[0], v[1]), pack2_bf16_rne(v[2], v[3]));
-                    }
-                    sum += __shfl_xor(sum, 16);
-                    sum += __shfl_xor(sum, 32);
-                    if (ei.g == 0)
-                        lr.sums[(long)(row0 / 128 + ei.wm) * lr.sums_pitch + col0 + cl] = sum;
-                }
-            };
-            if (row0 + BM <= m0)
-                stage(std::true_type{});
-            else
-                stage(std::false_type{});
-        } else if constexpr (ACT == kActRowScale) {
-            const EpiIds ei = epi_ids();
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
-                const f32x4 sc = *reinterpret_cast<const f32x4*>(lr.scale + row0 + rl);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                    const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
-                    float v[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = fmaf(acc[i][j][r], sc[r], bv);
-                    stage_rows4<1>(lds + rl * EP + cl * 2, EP, v);
-                }
-            }
-        } else if constexpr (YK != 0 && AWA == 0 && ACT != S2_ACT_SWIGLU) {
+        if constexpr (RES != 0) {
             const EpiIds ei = epi_ids();
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -493,11 +444,134 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                     const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
                     float v[4];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        v[r] = acc[i][j][r] + bv;
-                        if (ACT == S2_ACT_GELU) v[r] = gelu(v[r]);
+                    for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + bv;
+                    stage_rows4<1>(lds + rl * EP + cl * 2, EP, v);
+                }
+            }
+        }
+    };
+
+    // 16-bit outputs without a residual: every wave writes its own 128x64
+    // sub-tile, a quarter at a time, through two 4.5 KB LDS buffers of its own,
+    // so no wave waits for another.  A quarter's stores drain under the next
+    // one's arithmetic, and group 0 is done with its part while group 1 still
+    // issues its last MFMAs (no wave reads a stage by then: mainloop).  A store
+    // covers 128 bytes of 8 rows (kActExp: 256 bytes of 4 queries).  Assembling
+    // 512-byte rows from the four waves of a group instead took two barriers
+    // and left the stores to the end: MLP of the 720p video 1842 us, 1824 so;
+    // of 1485 rows 223 and 218; the VAE attention 533 and 508.
+    //
+    // Each stream's rows of the tile go through a buffer descriptor bounded by
+    // those rows, so the range check drops a row past its stream, and a chunk
+    // past n (an offset with bit 31 set: offsets are below 2^31, the launcher
+    // checks 256 rows of output), without a branch per store; the 8 rows of a
+    // store lie in one stream.  The output is not read again by this launch:
+    // the stores are non-temporal, leaving the L2 to the operand tiles.
+    auto wave_epilogue = [&]() {
+        if constexpr (YK != 0 && AWA == 0 && RES == 0 && ACT != S2_ACT_SWIGLU) {
+            const EpiIds ei = epi_ids();
+            const int ln = ei.tid & 63;
+            const int pitch = ny * 2;
+            uint8_t* mine = lds + (ei.wm * 4 + ei.wn) * kWaveStage;
+            if constexpr (ACT == kActExp) {
+                constexpr float kLog2e = 1.4426950408889634f;
+                constexpr int QP = 128 * 2 + 16;   // staged query row (bytes)
+                static_assert(2 * 16 * QP <= kWaveStage, "two quarters of 16 queries");
+                const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
+                    (char*)y0 + (long)col0 * pitch, (short)0, min(n - col0, BN) * pitch,
+                    kRawBufferFormat);
+                const int key = row0 + 128 * ei.wm + (ln & 15) * 8;
+                const uint32_t past = key < ny ? 0u : 0x80000000u;
+                auto quarters = [&](auto full_tag) {
+                    constexpr bool FULL = decltype(full_tag)::value;   // no key past m0
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        uint8_t* buf = mine + (j & 1) * 16 * QP;
+                        const int q0 = ei.wn * 64 + 16 * j;   // the quarter's first query
+                        const float ref = lr.ref[col0 + q0 + ei.l16];
+                        float sum = 0.f;
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const int rl = 16 * i + 4 * ei.g;
+                            float v[4];
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                v[r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], kLog2e, -ref));
+                                if (!FULL && row0 + 128 * ei.wm + rl + r >= m0) v[r] = 0.f;
+                            }
+                            sum += (v[0] + v[1]) + (v[2] + v[3]);
+                            *(uint2*)(buf + ei.l16 * QP + rl * 2) =
+                                make_uint2(pack2_bf16_rne(v[0], v[1]), pack2_bf16_rne(v[2], v[3]));
+                        }
+                        sum += __shfl_xor(sum, 16);
+                        sum += __shfl_xor(sum, 32);
+                        if (ei.g == 0)
+                            lr.sums[(long)(row0 / 128 + ei.wm) * lr.sums_pitch + col0 + q0 + ei.l16] = sum;
+                        asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int ql = (ln >> 4) + 4 * r;
+                            __builtin_amdgcn_raw_buffer_store_b128(
+                                *(const u32x4*)(buf + ql * QP + (ln & 15) * 16), rq,
+                                (uint32_t)((q0 + ql) * pitch + key * 2) | past, 0, kNonTemporal);
+                        }
+                        asm volatile("" ::: "memory");
                     }
-                    stage_rows4<YK>(lds + rl * EP + cl * 2, EP, v);
+                };
+                if (row0 + BM <= m0)
+                    quarters(std::true_type{});
+                else
+                    quarters(std::false_type{});
+            } else {
+                constexpr int RP = 64 * 2 + 16;   // staged row (bytes)
+                static_assert(2 * 32 * RP <= kWaveStage, "two quarters of 32 rows");
+                const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc(
+                    (char*)y0 + (long)row0 * pitch, (short)0, max(min(m0 - row0, BM), 0) * pitch,
+                    kRawBufferFormat);
+                const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(
+                    (char*)y1 + (long)(row0 - mv) * pitch, (short)0,
+                    row0 + BM > mv ? min(mv + m1 - row0, BM) * pitch : 0, kRawBufferFormat);
+                float bv[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
+                    bv[j] = (bias && col < n) ? bias[col] : 0.f;
+                }
+                const int cb = col0 + ei.wn * 64 + (ln & 7) * 8;   // the lane's 16-byte chunk
+                const uint32_t drop = cb < ny ? 0u : 0x80000000u;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    uint8_t* buf = mine + (c & 1) * 32 * RP;
+                    const int r0 = ei.wm * 128 + 32 * c;   // the quarter's first tile row
+#pragma unroll
+                    for (int ii = 0; ii < 2; ++ii) {
+                        const int rl = 16 * ii + 4 * ei.g;
+                        f32x4 sc;
+                        if constexpr (ACT == kActRowScale)
+                            sc = *reinterpret_cast<const f32x4*>(lr.scale + row0 + r0 + rl);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            float v[4];
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) {
+                                const float a = acc[2 * c + ii][j][r];
+                                v[r] = ACT == kActRowScale ? fmaf(a, sc[r], bv[j]) : a + bv[j];
+                                if (ACT == S2_ACT_GELU) v[r] = gelu(v[r]);
+                            }
+                            stage_rows4<YK>(buf + rl * RP + (16 * j + ei.l16) * 2, RP, v);
+                        }
+                    }
+                    asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const u32x4 sv = *(const u32x4*)(buf + (8 * r + (ln >> 3)) * RP + (ln & 7) * 16);
+                        const uint32_t off = (uint32_t)((r0 + 8 * r + (ln >> 3)) * pitch + cb * 2) | drop;
+                        if (row0 + r0 + 8 * r < mv)
+                            __builtin_amdgcn_raw_buffer_store_b128(sv, rs0, off, 0, kNonTemporal);
+                        else
+                            __builtin_amdgcn_raw_buffer_store_b128(sv, rs1, off, 0, kNonTemporal);
+                    }
+                    asm volatile("" ::: "memory");
                 }
             }
         }
@@ -521,7 +595,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     //             read step s               wait for its DMA
     //   group 1   MFMAs of step s - 1       read step s, wait for its DMA of
     //                                       step s + 1, DMA B of step s + 2
-    auto mainloop = [&](int kb, int ke, bool early) {
+    auto mainloop = [&](int kb, int ke, bool free) {
         const int grp = wave >> 2;
         const int wq = wave & 3;
         const int ld = lr.ld ? lr.ld : k;   // row pitch of x and of the weight
@@ -653,11 +727,11 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                                                                             acc[i][j], 0, 0, 0);
             __builtin_amdgcn_s_setprio(0);
             if (grp == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // A of step s + 1
-            barrier();
+            if (!(free && grp == 1 && s + 1 == steps)) barrier();
         }
-        // group 0's barrier matching group 1's last MFMA phase; with an early
-        // epilogue group 0 stages its rows first (epilogue)
-        if (grp == 0 && !early) barrier();
+        // group 0's barrier matching group 1's last MFMA phase (free: neither;
+        // group 1 read its last fragments before the barrier above)
+        if (grp == 0 && !free) barrier();
     };
 
     // The same sum for fp32 and fp16 activations (XK != 1), which are rounded
@@ -1179,7 +1253,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     };
 
     // y tile = act(acc + bias)
-    auto epilogue = [&](bool early) {
+    auto epilogue = [&]() {
         if constexpr (AWA != 0) {
             awa_epilogue();
             return;
@@ -1191,88 +1265,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         const EpiIds ei = epi_ids();
         if (YK && (ny & 7) == 0) {
             if constexpr (RES == 0) {
-                // Thread t of group g (waves 4g .. 4g + 3) stores 16-byte
-                // chunk t%32 of rows 128g + t/32 + 8c, all sixteen LDS reads
-                // before the first store.  Each stream's rows of the tile go
-                // through a buffer descriptor bounded by those rows, so the
-                // range check drops a row past its stream, and a chunk past
-                // n (an offset with bit 31 set: offsets are below 2^31, the
-                // launcher checks 256 rows of output), without a branch per
-                // store; a wave's two rows lie in one 8-row group, hence in
-                // one stream.  The output is not read again by this launch:
-                // the stores are non-temporal, leaving the L2 to the operand
-                // tiles.
-                //
-                // Early schedule (a whole tile): group 1's last MFMA phase
-                // reads no stage (its fragments are in registers, no DMA is
-                // in flight), so group 0 stages its rows 0-127 meanwhile and
-                // meets group 1 at the end of that phase (mainloop left that
-                // barrier to here); then group 0 stores while group 1 stages
-                // rows 128-255, and group 1 stores last.  Otherwise both
-                // groups stage, then store.  The barriers are plain s_barrier:
-                // group 0's stores need no wait before group 1 goes on.
-                const int pitch = ny * 2;
-                const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc(
-                    (char*)y0 + (long)row0 * pitch, (short)0, max(min(m0 - row0, BM), 0) * pitch,
-                    kRawBufferFormat);
-                const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(
-                    (char*)y1 + (long)(row0 - mv) * pitch, (short)0,
-                    row0 + BM > mv ? min(mv + m1 - row0, BM) * pitch : 0, kRawBufferFormat);
-                const int g0 = ei.wm;
-                const int t = ei.tid - 256 * g0;
-                const int ch = t & 31;
-                const int sub = t >> 5;
-                const int lw = ei.wn;   // wave within the group
-                const uint32_t drop = col0 + ch * 8 < ny ? 0u : 0x80000000u;
-                auto store_rows = [&]() {
-                    if constexpr (ACT == kActExp) {
-                        // 16-byte chunk t%16 of this group's 128 keys, queries
-                        // t/16 + 16c
-                        const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc(
-                            (char*)y0 + (long)col0 * pitch, (short)0, min(n - col0, BN) * pitch,
-                            kRawBufferFormat);
-                        const int key = row0 + 128 * g0 + (t & 15) * 8;
-                        const uint32_t past = key < ny ? 0u : 0x80000000u;
-                        u32x4 qv[16];
-#pragma unroll
-                        for (int c = 0; c < 16; ++c)
-                            qv[c] = *(const u32x4*)(lds + ((t >> 4) + 16 * c) * EP + 256 * g0 + (t & 15) * 16);
-#pragma unroll
-                        for (int c = 0; c < 16; ++c)
-                            __builtin_amdgcn_raw_buffer_store_b128(
-                                qv[c], rq, (uint32_t)(((t >> 4) + 16 * c) * pitch + key * 2) | past, 0,
-                                kNonTemporal);
-                        return;
-                    }
-                    u32x4 sv[16];
-#pragma unroll
-                    for (int c = 0; c < 16; ++c)
-                        sv[c] = *(const u32x4*)(lds + (128 * g0 + 8 * c + sub) * EP + ch * 16);
-#pragma unroll
-                    for (int c = 0; c < 16; ++c) {
-                        const int rl = 128 * g0 + 8 * c + sub;
-                        const uint32_t off = (uint32_t)(rl * pitch + col0 * 2 + ch * 16) | drop;
-                        if (row0 + 128 * g0 + 8 * c + 2 * lw < mv)
-                            __builtin_amdgcn_raw_buffer_store_b128(sv[c], rs0, off, 0, kNonTemporal);
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b128(sv[c], rs1, off, 0, kNonTemporal);
-                    }
-                };
-                auto plain_barrier = [] {
-                    __builtin_amdgcn_sched_barrier(0);
-                    asm volatile("s_barrier" ::: "memory");
-                    __builtin_amdgcn_sched_barrier(0);
-                };
-                const bool first_half = early && g0 == 0;
-                if (!early) plain_barrier();   // every wave is done reading the last stage
-                stage_own_rows();
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                if (first_half) {
-                    plain_barrier();
-                    store_rows();
-                }
-                plain_barrier();
-                if (!first_half) store_rows();
+                wave_epilogue();
             } else {
                 // the residual epilogue: thread t holds 16-byte chunk t%32 of
                 // tile rows t/32 + 16c
@@ -1384,14 +1377,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             __syncthreads();
         }
         bool finish = kb == 0 && ke == nk;
-        // the plain 16-bit epilogue of a whole tile without an activation runs
-        // early (see epilogue); with GELU the early schedule would serialise
-        // the two groups' VALU work, which otherwise shares the SIMDs
-        const bool early = AWA == 0 && RES == 0 && XK == 1 &&
-                           (ACT == S2_ACT_NONE || ACT == kActExp || ACT == kActRowScale) &&
-                           YK != 0 && (ny & 7) == 0 && finish;
+        // a whole tile that takes wave_epilogue: no wave meets another after
+        // the last MFMA phase, so the barrier there is left out
+        const bool free = AWA == 0 && RES == 0 && XK == 1 && ACT != S2_ACT_SWIGLU && YK != 0 &&
+                          (ny & 7) == 0 && finish;
         if constexpr (XK == 1)
-            mainloop(kb, ke, early);
+            mainloop(kb, ke, free);
         else
             mainloop_cvt(kb, ke);
         if (!finish) {
@@ -1463,7 +1454,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 finish = true;
             }
         }
-        if (finish) epilogue(early);
+        if (finish) epilogue();
         // every memory operation of this segment is complete: a real
         // s_waitcnt (not asm) lets the compiler's wait insertion know, so
         // it adds no vmcnt wait of its own inside the next main loop
