@@ -430,27 +430,6 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         return e;
     };
 
-    // acc + bias of this wave's rows of the tile as bf16 values in the LDS
-    // staging rows (pitch EP) of the residual epilogue
-    auto stage_own_rows = [&]() {
-        if constexpr (RES != 0) {
-            const EpiIds ei = epi_ids();
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int rl = ei.wm * 128 + 16 * i + 4 * ei.g;
-                    float v[4];
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = acc[i][j][r] + bv;
-                    stage_rows4<1>(lds + rl * EP + cl * 2, EP, v);
-                }
-            }
-        }
-    };
-
     // 16-bit outputs without a residual: every wave writes its own 128x64
     // sub-tile, a quarter at a time, through two 4.5 KB LDS buffers of its own,
     // so no wave waits for another.  A quarter's stores drain under the next
@@ -751,7 +730,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     //                            stage (s + 2) % 4, read last in step s - 2;
     //                            load A of step s + 4; wait for B of step s + 1
     //
-    // 3677 x 2560 by 2560 x 2560 from fp32: 104 us (150 tiles on 256 CUs), 262 us
+    // 3677 x 2560 by 2560 x 2560 from fp32: 101 us (150 tiles on 256 CUs), 262 us
     // with the 128 kernel, which staged A through registers one step ahead and
     // rounded it with integer operations; 15064 x 3072 by 9216 x 3072 from fp32
     // 1074 against 2775 us, 1038 us from fp16, 272 x 2560 by 2560 x 2560 50
@@ -1158,96 +1137,184 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         }
     };
 
-    // Residual epilogue: thread (sub, ch) holds the bf16 projection of
-    // columns col0 + 8 ch .. + 7 of tile rows sub + 16 c; all residual loads
-    // go out before the first store.  out may be x: each element is read and
-    // written by one thread.
-    auto residual_store = [&](const u32x4 (&sv)[16], int sub, int ch) {
+    // fp32 outputs in whole 16-byte chunks, as in wave_epilogue: a wave's rows
+    // leave 16 at a time, 256 bytes of 4 rows a store (in two halves of 128
+    // whole rows before: 3677 x 2560 by 2560 x 2560 from fp32 104 us, 101 so).
+    auto wave_epilogue_f32 = [&]() {
+        if constexpr (YK == 0 && AWA == 0 && RES == 0 && ACT != S2_ACT_SWIGLU) {
+            const EpiIds ei = epi_ids();
+            const int ln = ei.tid & 63;
+            constexpr int RP = 64 * 4 + 16;   // staged row (bytes)
+            static_assert(2 * 16 * RP <= kWaveStage, "two parts of 16 rows");
+            uint8_t* mine = lds + (ei.wm * 4 + ei.wn) * kWaveStage;
+            const int pitch = n * 4;
+            const __amdgpu_buffer_rsrc_t rs0 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)y0 + (long)row0 * pitch, (short)0, max(min(m0 - row0, BM), 0) * pitch,
+                kRawBufferFormat);
+            const __amdgpu_buffer_rsrc_t rs1 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)y1 + (long)(row0 - mv) * pitch, (short)0,
+                row0 + BM > mv ? min(mv + m1 - row0, BM) * pitch : 0, kRawBufferFormat);
+            float bv[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
+                bv[j] = (bias && col < n) ? bias[col] : 0.f;
+            }
+            const int cb = col0 + ei.wn * 64 + (ln & 15) * 4;   // the lane's 16-byte chunk
+            const uint32_t drop = cb < n ? 0u : 0x80000000u;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                uint8_t* buf = mine + (i & 1) * 16 * RP;
+                const int r0 = ei.wm * 128 + 16 * i;
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float v = acc[i][j][r] + bv[j];
+                        if (ACT == S2_ACT_GELU) v = gelu(v);
+                        *(float*)(buf + (4 * ei.g + r) * RP + (16 * j + ei.l16) * 4) = v;
+                    }
+                asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const u32x4 sv = *(const u32x4*)(buf + (4 * r + (ln >> 4)) * RP + (ln & 15) * 16);
+                    const uint32_t off = (uint32_t)((r0 + 4 * r + (ln >> 4)) * pitch + cb * 4) | drop;
+                    if (row0 + r0 + 4 * r < mv)
+                        __builtin_amdgcn_raw_buffer_store_b128(sv, rs0, off, 0, kNonTemporal);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b128(sv, rs1, off, 0, kNonTemporal);
+                }
+                asm volatile("" ::: "memory");
+            }
+        }
+    };
+
+    // Residual epilogue, as in wave_epilogue: a quarter's projection, rounded
+    // to bf16, is staged in the wave's own LDS while the residual of the next
+    // quarter is on its way; a lane then holds 4 columns of 8 rows.  out may be
+    // x: each element is read and written by one lane.  (Assembled over a
+    // workgroup and loaded in two halves before: MLP of 1485 rows 216 us, 210
+    // so; of the 720p video 1816 and 1803.)
+    auto wave_residual = [&]() {
         if constexpr (RES != 0) {
 #pragma clang fp contract(off)
-            const int col = col0 + ch * 8;
-            if (col >= n) return;
-            int cur = -1;
-            float g[8];
-            // two halves of eight rows: the half's residual loads (raw, two
-            // 16-byte chunks for fp32, one for 16-bit types) go out first
+            const EpiIds ei = epi_ids();
+            const int ln = ei.tid & 63;
+            constexpr int RP = 64 * 2 + 16;   // staged row (bytes)
+            uint8_t* mine = lds + (ei.wm * 4 + ei.wn) * kWaveStage;
+            const int es = res.x_kind == 0 ? 4 : 2;
+            const int pitch = n * es;
+            const int rows0 = max(min(m0 - row0, BM), 0);
+            const int rows1 = row0 + BM > mv ? min(mv + m1 - row0, BM) : 0;
+            const __amdgpu_buffer_rsrc_t rx0 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)res.x[0] + (long)row0 * pitch, (short)0, rows0 * pitch, kRawBufferFormat);
+            const __amdgpu_buffer_rsrc_t rx1 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)res.x[1] + (long)(row0 - mv) * pitch, (short)0, rows1 * pitch, kRawBufferFormat);
+            const __amdgpu_buffer_rsrc_t ro0 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)res.out[0] + (long)row0 * pitch, (short)0, rows0 * pitch, kRawBufferFormat);
+            const __amdgpu_buffer_rsrc_t ro1 = __builtin_amdgcn_make_buffer_rsrc(
+                (char*)res.out[1] + (long)(row0 - mv) * pitch, (short)0, rows1 * pitch, kRawBufferFormat);
+            const int sub = ln >> 4;
+            const int col = col0 + ei.wn * 64 + (ln & 15) * 4;   // n is a multiple of 8
+            const bool in = col < n;
+            const uint32_t drop = in ? 0u : 0x80000000u;
+            float bv[4];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                int loc[8];   // stream << 30 | row within the stream; -1: no row
-                u32x4 raw[8][2];
+            for (int j = 0; j < 4; ++j) {
+                const int c = col0 + ei.wn * 64 + 16 * j + ei.l16;
+                bv[j] = (bias && c < n) ? bias[c] : 0.f;
+            }
+            // 8-byte chunks of 16-bit residuals come in the first two words
+            auto load = [&](int c, u32x4 (&raw)[8]) {
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const int r = row0 + 16 * (8 * h + c) + sub;
-                    const int st = r < m0 ? 0 : (r >= mv && r < mv + m1 ? 1 : -1);
-                    const int local = st == 0 ? r : r - mv;
-                    loc[c] = st < 0 ? -1 : (st << 30) | local;
-                    if (st < 0) continue;
-                    const long e = (long)local * n + col;
-                    const void* xs = st ? res.x[1] : res.x[0];
+                for (int r = 0; r < 8; ++r) {
+                    const int rl = ei.wm * 128 + 32 * c + 4 * r;
+                    const uint32_t off = (uint32_t)((rl + sub) * pitch + col * es) | drop;
+                    const bool video = row0 + rl < mv;   // 8-row groups lie in one stream
                     if (res.x_kind == 0) {
-                        raw[c][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const float*)xs + e));
-                        raw[c][1] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const float*)xs + e + 4));
+                        raw[r] = video ? __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, kNonTemporal)
+                                       : __builtin_amdgcn_raw_buffer_load_b128(rx1, off, 0, kNonTemporal);
                     } else {
-                        raw[c][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((const uint16_t*)xs + e));
+                        const auto h = video ? __builtin_amdgcn_raw_buffer_load_b64(rx0, off, 0, kNonTemporal)
+                                             : __builtin_amdgcn_raw_buffer_load_b64(rx1, off, 0, kNonTemporal);
+                        raw[r][0] = h[0];
+                        raw[r][1] = h[1];
                     }
                 }
+            };
+            int cur = -1;
+            float g[4] = {0.f, 0.f, 0.f, 0.f};
+            u32x4 raw[2][8];
+            load(0, raw[0]);
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    if (loc[c] < 0) continue;
-                    const int st = loc[c] >> 30;
-                    const int local = loc[c] & 0x3fffffff;
-                    // the row's sample: the number of its stream's row ends
-                    // at or below it (the ends are read with uniform indices)
-                    int b = 0;
-                    for (int j = 0; j + 1 < res.rows.batch; ++j) {
-                        const int e = st ? res.rows.end[kAdaMaxBatch + j] : res.rows.end[j];
-                        if (local >= e) b = j + 1;
+            for (int c = 0; c < 4; ++c) {
+                if (c < 3) load(c + 1, raw[(c + 1) & 1]);
+                uint8_t* buf = mine + (c & 1) * 32 * RP;
+#pragma unroll
+                for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        float v[4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[r] = acc[2 * c + ii][j][r] + bv[j];
+                        stage_rows4<1>(buf + (16 * ii + 4 * ei.g) * RP + (16 * j + ei.l16) * 2, RP, v);
                     }
-                    const int key = st * kAdaMaxBatch + b;
-                    if (key != cur) {
+                asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const int rl = ei.wm * 128 + 32 * c + 4 * r;
+                    const bool video = row0 + rl < mv;
+                    const int local = row0 + rl + sub - (video ? 0 : mv);
+                    // the row's sample: the number of its stream's row ends at
+                    // or below it (the ends are read with uniform indices)
+                    int b = 0;
+                    for (int k2 = 0; k2 + 1 < res.rows.batch; ++k2) {
+                        const int e = video ? res.rows.end[k2] : res.rows.end[kAdaMaxBatch + k2];
+                        if (local >= e) b = k2 + 1;
+                    }
+                    const int key = (video ? 0 : kAdaMaxBatch) + b;
+                    if (key != cur && in) {
                         cur = key;
                         const float* ga = res.gate + (long)b * n + col;
-                        const float* gs = st ? res.gate_s[1] : res.gate_s[0];
+                        const float* gs = video ? res.gate_s[0] : res.gate_s[1];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) g[i] = gs ? ga[i] + gs[col + i] : ga[i];
+                        for (int i = 0; i < 4; ++i) g[i] = gs ? ga[i] + gs[col + i] : ga[i];
                     }
-                    float xv[8];
-                    if (res.x_kind == 0) {
+                    const u32x4 xr = raw[c & 1][r];
+                    const uint2 yw = *(const uint2*)(buf + (4 * r + sub) * RP + (ln & 15) * 8);
+                    float o[4];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) xv[i] = __uint_as_float(raw[c][i >> 2][i & 3]);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 8; ++i) {
-                            const uint16_t hv = (uint16_t)(raw[c][0][i >> 1] >> (16 * (i & 1)));
-                            xv[i] = res.x_kind == 1 ? bf16_to_f32(hv)
-                                                    : (float)__builtin_bit_cast(_Float16, hv);
-                        }
-                    }
-                    const u32x4 yw = sv[8 * h + c];
-                    float o[8];
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const uint32_t w = yw[i >> 1];
+                    for (int i = 0; i < 4; ++i) {
+                        const uint16_t hv = (uint16_t)(xr[i >> 1] >> (16 * (i & 1)));
+                        const float x = res.x_kind == 0   ? __uint_as_float(xr[i])
+                                        : res.x_kind == 1 ? bf16_to_f32(hv)
+                                                          : (float)__builtin_bit_cast(_Float16, hv);
+                        const uint32_t w = i >> 1 ? yw.y : yw.x;
                         const float y = __uint_as_float(i & 1 ? (w & 0xffff0000u) : (w << 16));
                         const float p = y * g[i];
-                        o[i] = xv[i] + p;
+                        o[i] = x + p;
                     }
-                    const long e = (long)local * n + col;
-                    void* os = st ? res.out[1] : res.out[0];
+                    const uint32_t off = (uint32_t)((rl + sub) * pitch + col * es) | drop;
                     if (res.x_kind == 0) {
-                        u32x4 a, b2;
+                        u32x4 ov;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            a[i] = __float_as_uint(o[i]);
-                            b2[i] = __float_as_uint(o[4 + i]);
-                        }
-                        __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>((float*)os + e));
-                        __builtin_nontemporal_store(b2, reinterpret_cast<u32x4*>((float*)os + e + 4));
+                        for (int i = 0; i < 4; ++i) ov[i] = __float_as_uint(o[i]);
+                        if (video)
+                            __builtin_amdgcn_raw_buffer_store_b128(ov, ro0, off, 0, kNonTemporal);
+                        else
+                            __builtin_amdgcn_raw_buffer_store_b128(ov, ro1, off, 0, kNonTemporal);
                     } else {
-                        store4(os, e, o[0], o[1], o[2], o[3], res.x_kind);
-                        store4(os, e + 4, o[4], o[5], o[6], o[7], res.x_kind);
+                        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+                        const u32x2 ov = res.x_kind == 1
+                                             ? u32x2{pack2_bf16_rne(o[0], o[1]), pack2_bf16_rne(o[2], o[3])}
+                                             : u32x2{pack2_f16_rne(o[0], o[1]), pack2_f16_rne(o[2], o[3])};
+                        if (video)
+                            __builtin_amdgcn_raw_buffer_store_b64(ov, ro0, off, 0, kNonTemporal);
+                        else
+                            __builtin_amdgcn_raw_buffer_store_b64(ov, ro1, off, 0, kNonTemporal);
                     }
                 }
+                asm volatile("" ::: "memory");
             }
         }
     };
@@ -1262,67 +1329,19 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             swiglu_epilogue();
             return;
         }
-        const EpiIds ei = epi_ids();
+        if constexpr (RES != 0) {
+            wave_residual();
+            return;
+        }
         if (YK && (ny & 7) == 0) {
-            if constexpr (RES == 0) {
-                wave_epilogue();
-            } else {
-                // the residual epilogue: thread t holds 16-byte chunk t%32 of
-                // tile rows t/32 + 16c
-                __syncthreads();   // every wave is done reading the last stage
-                stage_own_rows();
-                __syncthreads();
-                const int ch = ei.tid & 31;
-                const int sub = ei.tid >> 5;
-                u32x4 sv[16];
-#pragma unroll
-                for (int c = 0; c < 16; ++c)
-                    sv[c] = *(const u32x4*)(lds + (16 * c + sub) * EP + ch * 16);
-                residual_store(sv, sub, ch);
-            }
+            wave_epilogue();
             return;
         }
         if (!YK && (n & 3) == 0) {
-            // fp32: the same LDS staging in two halves of 128 rows (1 KB
-            // rows); the waves of row half h (wm == h) fill it, then all
-            // store 16-byte row chunks
-            constexpr int EF = BN * 4 + 16;   // fp32 row pitch (bytes)
-            static_assert(128 * EF <= LDS_BYTES, "fp32 half tile exceeds the LDS");
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                __syncthreads();   // the stage (h = 0) or the previous half is no longer read
-                if (ei.wm == h) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const int cl = ei.wn * 64 + 16 * j + ei.l16;
-                        const float bv = (bias && col0 + cl < n) ? bias[col0 + cl] : 0.f;
-#pragma unroll
-                        for (int i = 0; i < 8; ++i)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                float v = acc[i][j][r] + bv;
-                                if (ACT == S2_ACT_GELU) v = gelu(v);
-                                const int rl = 16 * i + 4 * ei.g + r;
-                                *(float*)(lds + rl * EF + cl * 4) = v;
-                            }
-                    }
-                }
-                __syncthreads();
-                // 128 rows x 1024 bytes: thread t stores chunk t%64 of rows
-                // t/64 + 8c
-#pragma unroll 4
-                for (int c = 0; c < 16; ++c) {
-                    const int rl = (ei.tid >> 6) + 8 * c;
-                    const int ch = ei.tid & 63;
-                    const int col = col0 + ch * 4;
-                    float* yr = (float*)out_row(h * 128 + rl);
-                    if (yr && col < n)
-                        __builtin_nontemporal_store(*(const u32x4*)(lds + rl * EF + ch * 16),
-                                                    (u32x4*)(yr + col));
-                }
-            }
+            wave_epilogue_f32();
             return;
         }
+        const EpiIds ei = epi_ids();
         // ragged n: direct stores
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1377,10 +1396,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             __syncthreads();
         }
         bool finish = kb == 0 && ke == nk;
-        // a whole tile that takes wave_epilogue: no wave meets another after
-        // the last MFMA phase, so the barrier there is left out
-        const bool free = AWA == 0 && RES == 0 && XK == 1 && ACT != S2_ACT_SWIGLU && YK != 0 &&
-                          (ny & 7) == 0 && finish;
+        // a whole tile whose waves write their own parts: no wave meets
+        // another after the last MFMA phase, so the barrier there is left out
+        const bool free = AWA == 0 && XK == 1 && ACT != S2_ACT_SWIGLU && finish &&
+                          (RES != 0 || (YK ? (ny & 7) == 0 : (n & 3) == 0));
         if constexpr (XK == 1)
             mainloop(kb, ke, free);
         else
