@@ -347,6 +347,11 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     constexpr int RB = BK * 2;        // LDS row bytes
     constexpr int EP = BN * 2 + 16;   // epilogue LDS row pitch (bytes)
     constexpr int LDS_BYTES = 2 * SB > BM * EP ? 2 * SB : BM * EP;
+    // row-tiles per raster group: 4 is 1-3% faster than 8 or 16 on a video's 85
+    // row-tiles.  (An image's 5 to 12 row-tiles in groups of about one height:
+    // 0.97 to 1.02 of these times over 4 to 20 row-tiles and five weight shapes,
+    // which is also how far the unchanged sizes spread.)
+    constexpr int GROUP = 4;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_BYTES];
     __shared__ int arrival;
     __shared__ QkvRow qrows[AWA ? BM : 1];
@@ -374,21 +379,11 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // tile holding the video tail also holds the first text rows.  Every
     // 8-row DMA group lies in one stream.
     int row0, col0;   // the current tile
-    // Row-tiles per raster group: 4 (1-3% faster than 8 or 16 on a video's 85
-    // row-tiles, 1% than 5), but the few row-tiles of an image in groups of
-    // about one height, whose last sweep reads the weight for as many rows as
-    // the others: 7 as one group instead of 4 + 3 (MLP of 1549 rows 210 -> 207
-    // us), 10 as 5 + 5 instead of 4 + 4 + 2 (block of 2368 rows 492 -> 487).
-    // SwiGLU (10 row-tiles 147.4 against 146.5 us) and the converting loop,
-    // which the height in a register cost 3%, keep 4.
-    const int group = ACT != S2_ACT_SWIGLU && XK == 1 && mtiles > 4 && mtiles <= 12
-                          ? (mtiles + mtiles / 4 - 1) / (mtiles / 4)
-                          : 4;
     auto set_tile = [&](int t) {
-        // grouped raster: `group` m-tiles share each sweep over the n-tiles
-        const int group_size = group * ntiles;
-        const int first_m = (t / group_size) * group;
-        const int gm = min(mtiles - first_m, group);
+        // grouped raster: GROUP m-tiles share each sweep over the n-tiles
+        const int group_size = GROUP * ntiles;
+        const int first_m = (t / group_size) * GROUP;
+        const int gm = min(mtiles - first_m, GROUP);
         const int mt = first_m + (t % group_size) % gm;
         const int nt = (t % group_size) / gm;
         row0 = mt * BM;
