@@ -254,8 +254,11 @@ __global__ void __launch_bounds__(kThreads) cfg_stats_kernel(const float* __rest
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             n += min(max(count - (base + j * 1024 + (tid >> 6) * 256), 0L), 256L);
-        const double inv = 1.0 / (double)max(n, 1L);
-        const double mp = sp * inv, mg = sg * inv;
+        // quotients, not products with 1 / n: the mean of equal values is then
+        // exactly their value, and a constant cfg has the deviation 0 that
+        // leaves it unscaled
+        const double dn = (double)max(n, 1L);
+        const double mp = sp / dn, mg = sg / dn;
         double qp = 0.0, qg = 0.0;
 #pragma unroll
         for (int e = 0; e < 16; ++e)

@@ -122,6 +122,17 @@ def test_apply_cfg_zero_spread_and_nan():
     assert np.isnan(ref).all() and np.isnan(got).all()
 
 
+@pytest.mark.parametrize("count", [2, 49, 256, 257, 1000, 4096 + 98, 3 * 4096 + 1024 + 49])
+def test_apply_cfg_constant_predictions(count):
+    """Equal elements have standard deviation exactly 0, which leaves cfg
+    unscaled; a mean that is off in its last bit would give two deviations of
+    an ulp instead, and any quotient of them as the factor."""
+    for p, n in ((0.3, 0.1), (0.7, -0.9), (1e-3, 3.3)):
+        pos, neg = np.full(count, p, np.float32), np.full(count, n, np.float32)
+        got = _host(capi.apply_cfg(_cuda(pos), _cuda(neg), 6.5, 0.7))
+        assert np.array_equal(got, oracle.apply_cfg(pos, neg, 6.5, 0.0))
+
+
 @pytest.mark.parametrize("tokens", [1, 255, 257, 86400])
 def test_euler_step_bit_exact(tokens):
     g = np.random.default_rng(tokens)
