@@ -75,7 +75,7 @@ struct LinearRows {
 };
 // y[r][c] = exp2(log2(e) (q keys^T)[r][c] - ref[r]) for c < n, 0 for n <= c <
 // pitch, bf16, over m rows of q and n keys; sums[t][r] the fp32 sum of row r's
-// values in columns [128 t, + 128)
+// bf16 values in columns [128 t, + 128)
 hipError_t launch_linear_exp(const uint16_t* q, int m, const uint16_t* keys, int n, int k,
                              uint16_t* y, const LinearRows& lr, hipStream_t stream);
 // y = (x W^T) scale[r] + bias, bf16 [m][n], n % 8 == 0

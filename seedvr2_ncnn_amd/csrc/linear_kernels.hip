@@ -328,7 +328,8 @@ __device__ __forceinline__ void stage_rows4(uint8_t* p, int pitch, const float (
 // Epilogues of the VAE attention's products (one stream, bf16 output):
 //   kActExp       rows are keys, columns queries: y[query][key] = exp(acc -
 //                 reference of the query), zeros for keys past m0 up to the
-//                 row pitch, and per 128 keys the fp32 sums of a query's values.
+//                 row pitch, and per 128 keys the fp32 sums of a query's values
+//                 as stored.
 //                 A lane holds four consecutive keys of a query: packed
 //                 conversions, 8-byte LDS writes and sums within the lane
 //   kActRowScale  y = acc * (scale of the row) + bias
@@ -480,9 +481,15 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                                 v[r] = __builtin_amdgcn_exp2f(fmaf(acc[i][j][r], kLog2e, -ref));
                                 if (!FULL && row0 + 128 * ei.wm + rl + r >= m0) v[r] = 0.f;
                             }
-                            sum += (v[0] + v[1]) + (v[2] + v[3]);
-                            *(uint2*)(buf + ei.l16 * QP + rl * 2) =
-                                make_uint2(pack2_bf16_rne(v[0], v[1]), pack2_bf16_rne(v[2], v[3]));
+                            // the sums are of the rounded values: the weights
+                            // that the product with V uses then add up to one,
+                            // and a row with few large ones keeps the precision
+                            // that rounding normalised probabilities gives
+                            const uint32_t w0 = pack2_bf16_rne(v[0], v[1]);
+                            const uint32_t w1 = pack2_bf16_rne(v[2], v[3]);
+                            sum += (__uint_as_float(w0 << 16) + __uint_as_float(w0 & 0xffff0000u)) +
+                                   (__uint_as_float(w1 << 16) + __uint_as_float(w1 & 0xffff0000u));
+                            *(uint2*)(buf + ei.l16 * QP + rl * 2) = make_uint2(w0, w1);
                         }
                         sum += __shfl_xor(sum, 16);
                         sum += __shfl_xor(sum, 32);

@@ -119,6 +119,32 @@ def test_mha_long_sequences(seq, heads, kind):
     assert_close(got[rows], oracle.mha(x, heads, *ws, rows=rows, threads=16, fast=True))
 
 
+@pytest.mark.parametrize("seq,heads", [(1024, 1), (4096, 2)])
+def test_mha_weights_of_a_row_sum_to_one(seq, heads):
+    """Values that are the same for every key come back as they are: what a row's
+    weights are divided by is the sum of the bf16 weights themselves.  Scores
+    of standard deviation 2.5, so that a few keys hold most of a row.  The
+    output projection averages 512 channels of different values, so the
+    rounding of the concatenated heads (rms 2^-9 / sqrt 3 a channel) is left with
+    5e-5; eight of these."""
+    import torch
+    g = np.random.default_rng(seq)
+    e = 512
+    x = g.standard_normal((seq, e)).astype(np.float32)
+    x[:, 0] = 1.0
+    ws = _weights(g, e, e)
+    ws[0] *= 2.5
+    c = bf16_round(g.uniform(1, 2, e).astype(np.float32))
+    ws[4] = np.zeros((e, e), np.float32)
+    ws[4][:, 0] = c
+    ws[5] = np.zeros(e, np.float32)
+    ws[6] = np.tile(bf16_round((1 / (e * c)).astype(np.float32)), (e, 1))
+    ws[7] = np.zeros(e, np.float32)
+    want = float(ws[6][0].astype(np.float64) @ c)
+    got = _run(_device(heads, ws), bf16_round(x), dtype=torch.bfloat16, out_dtype=torch.float32)
+    assert np.abs(got.astype(np.float64) / want - 1).max() <= 4e-4
+
+
 def test_mha_long_sequence_nan_reaches_every_row():
     g = np.random.default_rng(3)
     x = g.standard_normal((4700, 64)).astype(np.float32)
