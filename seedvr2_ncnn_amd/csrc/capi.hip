@@ -1566,8 +1566,8 @@ int s2_mha_forward(const s2_mha_config* config, const void* prepared, const void
             lr.scale = (const float*)(ws + w.scale);
             int* general = (int*)(ws + w.general);
             lr.ld = ld;
-            S2_HIP(s2::launch_mha_reference(q, kh, ld, seq, D, w.pitch, (float*)(ws + w.stats),
-                                            (float*)(ws + w.ref), general, st));
+            S2_HIP(s2::launch_mha_reference(q, kh, ld, vt, w.lp, seq, D, w.pitch,
+                                            (float*)(ws + w.stats), (float*)(ws + w.ref), general, st));
             lr.gate = general;
             lr.gate_want = 0;
             S2_HIP(s2::launch_linear_exp(q, seq, kh, seq, D, p, lr, st));

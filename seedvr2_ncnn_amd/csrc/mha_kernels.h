@@ -21,11 +21,12 @@ hipError_t launch_mha_softmax(const float* s, long ld_s, int rows, int cols, int
                               uint16_t* p, const int* gate, hipStream_t stream);
 // The exponentials' reference of each row of q k^T (bf16 rows of width d and
 // pitch ld, multiples of 8): ref[0, pitch), pitch >= rows a multiple of 256,
-// and *general = 1 when it does not cover every row, else 0; stats: 3 * pitch
-// floats of scratch, 16-byte aligned
-hipError_t launch_mha_reference(const uint16_t* q, const uint16_t* k, int ld, int rows, int d,
-                                int pitch, float* stats, float* ref, int* general,
-                                hipStream_t stream);
+// and *general = 1 when it does not cover every row or the values vt [d][lp]
+// (rows rounded up to 64; rows >= 64), else 0; stats: 3 * pitch floats of
+// scratch, 16-byte aligned
+hipError_t launch_mha_reference(const uint16_t* q, const uint16_t* k, int ld, const uint16_t* vt,
+                                int lp, int rows, int d, int pitch, float* stats, float* ref,
+                                int* general, hipStream_t stream);
 // scale[0, pitch): 1 / sum over parts of sums[part][row], or 1 when *general;
 // pitch % 64 == 0
 hipError_t launch_mha_row_scale(const float* sums, int parts, int pitch, const int* general,

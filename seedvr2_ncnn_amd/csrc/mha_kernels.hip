@@ -53,17 +53,28 @@ __global__ __launch_bounds__(256) void mha_stage_kernel(const void* __restrict__
 //
 // The scores of row r are bounded by B_r = |q_r| max_j |k_j| (log2 domain,
 // with 2^-6 of slack for the products' rounding).  Their exponentials are
-// taken relative to c_r = max(0, B_r - 80): no value exceeds 2^80, so the sums
-// of a row and of its product with V stay finite, and as long as the row's
-// largest score lies within 180 of B_r its probabilities stay above 2^-100,
-// with 2^-26 of them still normal numbers.  A row's own key shows that: the
-// reference is good for a head when q_r k_r >= B_r - 180 for every row.
-// Otherwise (also for non-finite operands) `general` sends the head through
-// fp32 scores and the softmax pass.
+// taken relative to c_r = max(0, B_r - 80): no value exceeds 2^80, and a
+// row's largest one is at least 2^-70 if its score lies within 150 of B_r,
+// with 2^-26 of it still 30 powers of two above the smallest normal number.  A
+// row's own key shows that: the reference is good for a head when q_r k_r >=
+// B_r - 150 for every row.  The product with V is divided by the row's sum
+// afterwards, so V has to leave it room: with every |v| at most 2^24 (and 2^21
+// keys) its sums stay below 2^125, and with one of at least 2^-30 in every run
+// of d values of V^T (or none but zeros) no channel's sums leave the normal
+// numbers.  Otherwise (also for non-finite operands) `general` sends the head
+// through fp32 scores and the softmax pass, whose weights are normalised
+// before V meets them.  (With no look at V, values of 1e30 came out as
+// infinity where every score was near its bound; it costs 1.5 us of 490 for
+// 14,400 tokens.)
+constexpr float kRefBelow = 80.f, kRefSpan = 150.f;
+constexpr uint32_t kValueMax = 0x4b800000u, kValueMin = 0x30800000u;   // 2^24, 2^-30
 
-// |q_r|^2, |k_r|^2 and q_r k_r, one wave a row (row pitch ld); clears the flag
+// |q_r|^2, |k_r|^2 (NaN where V is out of range) and q_r k_r, one wave a row
+// (row pitch ld); clears the flag.  The wave also looks at run r of d values of
+// V^T [d][lp], and at run rows + r, of the padding, where there is one.
 __global__ __launch_bounds__(256) void mha_norms_kernel(const uint16_t* __restrict__ q,
                                                         const uint16_t* __restrict__ k, int ld,
+                                                        const uint16_t* __restrict__ vt, int lp,
                                                         int rows, int d, int pitch,
                                                         float* __restrict__ stats,
                                                         int* __restrict__ general) {
@@ -72,10 +83,20 @@ __global__ __launch_bounds__(256) void mha_norms_kernel(const uint16_t* __restri
     const int lane = threadIdx.x & 63;
     if (r >= rows) return;
     float qq = 0.f, kk = 0.f, qk = 0.f;
+    // magnitudes as fp32 bits: they order like the values, infinity and NaN on top
+    uint32_t vm = 0u;
+    auto magnitudes = [&](uint4 u) {
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            vm = max(vm, max((w[e] << 16) & 0x7fff0000u, w[e] & 0x7fff0000u));
+    };
     for (int c = lane * 8; c < d; c += 512) {
+        const uint4 u = *reinterpret_cast<const uint4*>(vt + (long)r * d + c);
         float a[8], b[8];
         load8(q + (long)r * ld + c, a);
         load8(k + (long)r * ld + c, b);
+        magnitudes(u);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             qq = fmaf(a[e], a[e], qq);
@@ -88,10 +109,20 @@ __global__ __launch_bounds__(256) void mha_norms_kernel(const uint16_t* __restri
         qq += __shfl_xor(qq, off);
         kk += __shfl_xor(kk, off);
         qk += __shfl_xor(qk, off);
+        vm = max(vm, (uint32_t)__shfl_xor((int)vm, off));
+    }
+    bool fits = vm <= kValueMax && (vm == 0u || vm >= kValueMin);
+    if (rows + r < lp) {   // lp < rows + 64 <= 2 rows
+        vm = 0u;
+        for (int c = lane * 8; c < d; c += 512)
+            magnitudes(*reinterpret_cast<const uint4*>(vt + (long)(rows + r) * d + c));
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) vm = max(vm, (uint32_t)__shfl_xor((int)vm, off));
+        fits = fits && vm <= kValueMax && (vm == 0u || vm >= kValueMin);
     }
     if (lane == 0) {
         stats[r] = qq;
-        stats[pitch + r] = kk;
+        stats[pitch + r] = fits ? kk : __uint_as_float(0x7fc00000u);
         stats[2 * pitch + r] = qk;
     }
 }
@@ -118,7 +149,7 @@ __global__ __launch_bounds__(256) void mha_reference_kernel(const float* __restr
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if (i + e >= rows) continue;
-            bad |= !(v[e] <= 3.0e38f);   // also for NaN
+            bad |= !(v[e] <= 3.0e38f);   // also for NaN (mha_norms_kernel's too)
             m = fmaxf(m, v[e]);
         }
     }
@@ -129,8 +160,8 @@ __global__ __launch_bounds__(256) void mha_reference_kernel(const float* __restr
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
     const float b = sqrtf(qq) * sqrtf(m) * (kLog2e * (1.f + 0.015625f));
     const bool in = r < rows;
-    bad |= in && !(own >= b - 180.f);
-    ref[r] = in ? fmaxf(b - 80.f, 0.f) : 0.f;
+    bad |= in && !(own >= b - kRefSpan);
+    ref[r] = in ? fmaxf(b - kRefBelow, 0.f) : 0.f;
     if (__any(bad) && (t & 63) == 0)
         __hip_atomic_store(general, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -308,11 +339,11 @@ hipError_t launch_mha_stage(const void* x, int kind, int rows, int rows_padded, 
     return hipGetLastError();
 }
 
-hipError_t launch_mha_reference(const uint16_t* q, const uint16_t* k, int ld, int rows, int d,
-                                int pitch, float* stats, float* ref, int* general,
-                                hipStream_t stream) {
-    mha_norms_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, stream>>>(q, k, ld, rows, d, pitch, stats,
-                                                                     general);
+hipError_t launch_mha_reference(const uint16_t* q, const uint16_t* k, int ld, const uint16_t* vt,
+                                int lp, int rows, int d, int pitch, float* stats, float* ref,
+                                int* general, hipStream_t stream) {
+    mha_norms_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, stream>>>(q, k, ld, vt, lp, rows, d,
+                                                                     pitch, stats, general);
     mha_reference_kernel<<<(unsigned)(pitch / 256), 256, 0, stream>>>(stats, rows, pitch, ref, general);
     return hipGetLastError();
 }

@@ -145,6 +145,27 @@ def test_mha_weights_of_a_row_sum_to_one(seq, heads):
     assert np.abs(got.astype(np.float64) / want - 1).max() <= 4e-4
 
 
+# (constant channel of q and k, the same channel in both, size of the values):
+# scores at their bound, with values that a sum of unnormalised weights has no
+# room for; scores about 170 and 125 powers of two below it, with values whose
+# products with weights that small are, or nearly are, no normal numbers
+@pytest.mark.parametrize("const,same,size", [(40, True, 1e6), (40, True, 1e12), (40, True, 1e30),
+                                             (29, False, 1e-16), (25, False, 1e-7)])
+def test_mha_large_and_small_values(const, same, size):
+    g = np.random.default_rng(int(const + np.log10(size) + 50))
+    x = g.standard_normal((1100, 64)).astype(np.float32)
+    ws = _weights(g, 64, 64)
+    for i, c in ((0, 0), (2, 0 if same else 1)):
+        ws[i][:2] = 0
+        ws[i + 1][:2] = 0
+        ws[i + 1][c] = const
+    for i in (4, 5):
+        ws[i] = (ws[i] * size).astype(np.float32)
+    ws[6] = (ws[6] / size).astype(np.float32)
+    rows = np.arange(0, 1100, 37).astype(np.int32)
+    assert_close(_run(_device(1, ws), x)[rows], oracle.mha(x, 1, *ws, rows=rows, threads=16))
+
+
 def test_mha_long_sequence_nan_reaches_every_row():
     g = np.random.default_rng(3)
     x = g.standard_normal((4700, 64)).astype(np.float32)
