@@ -312,7 +312,8 @@ S2_API int s2_copy_2d(const void* src, s2_dtype src_dtype, long src_stride, void
  * with the gate and up rows interleaved in blocks of 128 (rows 256j ..
  * 256j+127 are gate rows 128j .., rows 256j+128 .. 256j+255 up rows 128j ..;
  * s2_swiglu_pack_weight builds it), bias likewise [2n] or NULL; n (the
- * output width) a multiple of 128, bf16 activations, k a multiple of 64. */
+ * output width) a multiple of 128 below 2^20, bf16 activations, k a multiple
+ * of 64 below 2^22. */
 S2_API int s2_shared_linear_forward(const void* x_video, int m_video, const void* x_text, int m_text,
                              s2_dtype x_dtype, const uint16_t* weight, const float* bias,
                              int n, int k, int activation,

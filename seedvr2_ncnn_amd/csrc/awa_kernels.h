@@ -35,6 +35,12 @@ hipError_t launch_awa_qkv(const s2_awa_plan& plan, const uint16_t* x_video, cons
 hipError_t launch_cast_f32_bf16(const float* src, uint16_t* dst, size_t n, hipStream_t stream);
 hipError_t launch_gelu(const void* x, void* y, size_t n, int kind, hipStream_t stream);
 hipError_t launch_cast_bf16_f32(const uint16_t* src, float* dst, size_t n, hipStream_t stream);
+// Shapes of the SwiGLU projection (output width n, weight [2n][k]): only the
+// 256-tile kernel forms the gate, whose buffer offsets are 32-bit.
+inline bool swiglu_shape_ok(int n, int k) {
+    return k % 64 == 0 && n % 128 == 0 && (long)256 * k * 2 <= 0x7fffffffL &&
+           (long)256 * 2 * n * 4 <= 0x7fffffffL;
+}
 // Grouped y_s = act(x_s W^T + b) over the video and text streams.
 hipError_t launch_shared_linear(const void* x0, int m0, const void* x1, int m1, int x_kind,
                                 const uint16_t* w, const float* bias, int n, int k, int act,

@@ -876,9 +876,9 @@ static int linear_args_ok(const void* x_video, int m_video, const void* x_text, 
     if (activation != S2_ACT_NONE && activation != S2_ACT_GELU && activation != S2_ACT_SWIGLU)
         return fail(S2_ERR_INVALID, "unknown activation");
     if (!dtype_ok(x_dtype) || !dtype_ok(y_dtype)) return fail(S2_ERR_INVALID, "unsupported dtype");
-    if (activation == S2_ACT_SWIGLU &&
-        (x_dtype != S2_DTYPE_BF16 || k % 64 != 0 || n % 128 != 0 || (long)256 * k * 2 > 0x7fffffffL))
-        return fail(S2_ERR_INVALID, "SwiGLU needs bf16 activations, k % 64 == 0 and n % 128 == 0");
+    if (activation == S2_ACT_SWIGLU && (x_dtype != S2_DTYPE_BF16 || !s2::swiglu_shape_ok(n, k)))
+        return fail(S2_ERR_INVALID,
+                    "SwiGLU needs bf16 activations, k % 64 == 0, n % 128 == 0 and n < 2^20");
     const size_t xe = dtype_bytes(x_dtype);
     if (((uintptr_t)x_video) % (8 * xe) || ((uintptr_t)x_text) % (8 * xe) ||
         ((uintptr_t)weight) % 16 || ((uintptr_t)y_video) % 16 || ((uintptr_t)y_text) % 16)

@@ -1694,15 +1694,19 @@ static hipError_t linear_impl(const void* x0, int m0, const void* x1, int m1, co
             ntiles, sk, AwaQkvArgs{}, LinearResidual{}, LinearRows{});
         return hipGetLastError();
     }
-    const int mt0 = (m0 + 127) / 128;
-    const int mt1 = (m1 + 127) / 128;
-    const int ntiles = (n + 127) / 128;
-    const int mtiles = mt0 + mt1;
-    const long blocks = (long)mtiles * ntiles;
-    if (blocks == 0) return hipSuccess;
-    shared_linear_kernel<TX, YK, ACT><<<(unsigned)blocks, 256, 0, stream>>>(
-        (const TX*)x0, m0, (const TX*)x1, m1, w, bias, n, k, y0, y1, mt0, mtiles, ntiles);
-    return hipGetLastError();
+    if constexpr (ACT == S2_ACT_SWIGLU) {
+        return hipErrorInvalidValue;   // the 128 kernel has no gate
+    } else {
+        const int mt0 = (m0 + 127) / 128;
+        const int mt1 = (m1 + 127) / 128;
+        const int ntiles = (n + 127) / 128;
+        const int mtiles = mt0 + mt1;
+        const long blocks = (long)mtiles * ntiles;
+        if (blocks == 0) return hipSuccess;
+        shared_linear_kernel<TX, YK, ACT><<<(unsigned)blocks, 256, 0, stream>>>(
+            (const TX*)x0, m0, (const TX*)x1, m1, w, bias, n, k, y0, y1, mt0, mtiles, ntiles);
+        return hipGetLastError();
+    }
 }
 
 template <typename TX, int YK>
@@ -1710,11 +1714,11 @@ static hipError_t linear_act(int act, const void* x0, int m0, const void* x1, in
                              const uint16_t* w, const float* bias, int n, int k, void* y0,
                              void* y1, hipStream_t stream, SkSource src) {
     if (act == S2_ACT_SWIGLU) {
-        // bf16 activations on the 256-tile path only (the caller checks);
-        // n is the output width, the weight has 2n interleaved rows
+        // bf16 activations on the 256-tile path only (the caller checks), whose
+        // epilogue it is; n is the output width, the weight has 2n interleaved
+        // rows
         if constexpr (std::is_same<TX, uint16_t>::value) {
-            if (k % 64 != 0 || n % 128 != 0 || (long)256 * k * 2 > 0x7fffffffL)
-                return hipErrorInvalidValue;
+            if (!swiglu_shape_ok(n, k)) return hipErrorInvalidValue;
             return linear_impl<TX, YK, S2_ACT_SWIGLU>(x0, m0, x1, m1, w, bias, 2 * n, k, y0, y1,
                                                       stream, src);
         }

@@ -77,6 +77,17 @@ def test_shared_linear_validates_before_the_device():
                                       None) == capi.S2_ERR_INVALID
 
 
+@pytest.mark.parametrize("entry", ["s2_shared_linear_forward", "s2_shared_linear_forward_noalloc"])
+@pytest.mark.parametrize("n,k", [(1 << 20, 64), ((1 << 20) + 128, 128), ((1 << 30) + 128, 64),
+                                 (128, 1 << 22)])
+def test_swiglu_refuses_widths_beyond_the_kernel_that_forms_the_gate(entry, n, k):
+    # (any other kernel would store 2n raw columns into rows of n)
+    dummy = ctypes.c_void_p(256)
+    assert getattr(capi.lib(), entry)(dummy, 4, None, 0, capi.DTYPE_BF16, dummy, None, n, k,
+                                      capi.ACT_SWIGLU, dummy, None, capi.DTYPE_BF16,
+                                      None) == capi.S2_ERR_INVALID
+
+
 # ---- AdaptiveWindowAttention layer surface -----------------------------------------
 
 HEADS, D, PAIRS = 2, 64, 10
