@@ -306,7 +306,13 @@ S2_API int s2_copy_2d(const void* src, s2_dtype src_dtype, long src_stride, void
  * tiles are split along k over several workgroups, which meet in the
  * stream's scratch of partial tiles (one 256 KB slot per compute unit, 64 MB
  * on MI355X, plus counters; see s2_stream_scratch_acquire).  Calls on
- * different streams therefore never share scratch and may run concurrently. *
+ * different streams therefore never share scratch and may run concurrently.
+ * That holds for every x_dtype where k is a multiple of 64 (other k are never
+ * split).  A stream whose scratch does not exist yet cannot get it while it is
+ * capturing a graph: bf16 calls that would split fail there, fp32 and fp16
+ * ones run unsplit (an fp32 sum in another order).  A captured call keeps the
+ * stream's scratch: replay it where it does not overlap that stream's calls.
+ *
  * activation S2_ACT_SWIGLU (v3 graphs' MLP, seedvr2_pipeline.cpp:434-438):
  * y = silu(x Wg^T + bg) * (x Wu^T + bu) in one launch.  weight is [2n][k]
  * with the gate and up rows interleaved in blocks of 128 (rows 256j ..

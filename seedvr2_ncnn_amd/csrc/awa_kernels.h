@@ -41,10 +41,14 @@ inline bool swiglu_shape_ok(int n, int k) {
     return k % 64 == 0 && n % 128 == 0 && (long)256 * k * 2 <= 0x7fffffffL &&
            (long)256 * 2 * n * 4 <= 0x7fffffffL;
 }
-// Grouped y_s = act(x_s W^T + b) over the video and text streams.
+// Grouped y_s = act(x_s W^T + b) over the video and text streams.  On a
+// capturing stream without split-k scratch bf16 activations fail where their
+// last wave would be split; with optional_split, and fp32 and fp16 ones, run
+// unsplit.
 hipError_t launch_shared_linear(const void* x0, int m0, const void* x1, int m1, int x_kind,
                                 const uint16_t* w, const float* bias, int n, int k, int act,
-                                void* y0, void* y1, int y_kind, hipStream_t stream);
+                                void* y0, void* y1, int y_kind, hipStream_t stream,
+                                bool optional_split = false);
 // The same with the split-k scratch in a static device array: no allocation.
 hipError_t launch_shared_linear_noalloc(const void* x0, int m0, const void* x1, int m1,
                                         int x_kind, const uint16_t* w, const float* bias, int n,

@@ -1539,13 +1539,14 @@ int s2_mha_forward(const s2_mha_config* config, const void* prepared, const void
         const long wo_h = (long)h * D * Q;
         // q_h = x Wq_h^T + bq_h (scale folded in), k_h likewise: [lp][D]; with
         // one head and no gap between the two weights and biases, one product
-        // makes [lp][q | k]
+        // makes [lp][q | k] (whose tail may be split where the two products'
+        // are not: only if there is scratch for it)
         const bool joint = w.fused && m.wk == (size_t)E * Q * 2 && m.bk - m.bq == (size_t)E * 4 && H == 1;
         const int ld = joint ? 2 * D : D;
         const uint16_t* kh = joint ? q + D : k;
         if (joint) {
             S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wq, bq, 2 * D, Q, S2_ACT_NONE,
-                                            q, nullptr, kBF, st));
+                                            q, nullptr, kBF, st, true));
         } else {
             S2_HIP(s2::launch_shared_linear(xp, w.lp, nullptr, 0, kBF, wq + wo_h, bq + h * D, D, Q,
                                             S2_ACT_NONE, q, nullptr, kBF, st));

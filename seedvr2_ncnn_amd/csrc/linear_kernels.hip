@@ -1624,8 +1624,10 @@ __global__ void zero_counters_kernel(int* counters, int n) {
 // Where the split-k tail keeps its partial tiles: the calling stream's own
 // allocation (stream_scratch), or, for the no-allocation entry point, the
 // static `scratch` array (whose counters are cleared before every launch
-// that uses them, since a call keeps whatever the last one left).
-enum class SkSource { kStream, kStatic };
+// that uses them, since a call keeps whatever the last one left).  kOptional is
+// the stream's where there is one or one can be made, else no split: for calls
+// that have to work on a capturing stream that nobody owns.
+enum class SkSource { kStream, kOptional, kStatic };
 
 // Split-k tail of a launch of `tiles` 256x256 tiles with nk 64-k steps:
 // when the last wave of tiles would leave more than 3% of the workgroup
@@ -1661,8 +1663,14 @@ static hipError_t plan_sk_tail(long tiles, int nk, SkSource source, hipStream_t 
             e = hipGetLastError();
             if (e != hipSuccess) return e;
         } else {
-            e = stream_scratch(kScratchSplitK, stream, sk_scratch_bytes(G), &base);
+            e = source == SkSource::kOptional
+                    ? stream_scratch_optional(kScratchSplitK, stream, sk_scratch_bytes(G), &base)
+                    : stream_scratch(kScratchSplitK, stream, sk_scratch_bytes(G), &base);
             if (e != hipSuccess) return e;
+            if (!base) {
+                *out = SkTail{(int)tiles, 0, 0, nullptr, nullptr};
+                return hipSuccess;
+            }
             sk.slots = (float*)base;
             sk.counters = (int*)((char*)base + (size_t)G * kSlotFloats * 4);
         }
@@ -1753,9 +1761,12 @@ static hipError_t linear_dispatch(const void* x0, int m0, const void* x1, int m1
 
 hipError_t launch_shared_linear(const void* x0, int m0, const void* x1, int m1, int x_kind,
                                 const uint16_t* w, const float* bias, int n, int k, int act,
-                                void* y0, void* y1, int y_kind, hipStream_t stream) {
+                                void* y0, void* y1, int y_kind, hipStream_t stream,
+                                bool optional_split) {
+    // (fp32 and fp16 activations can do without the scratch: they took the
+    // 128-tile kernel, which has no split, until the 256-tile one converted them)
     return linear_dispatch(x0, m0, x1, m1, x_kind, w, bias, n, k, act, y0, y1, y_kind, stream,
-                           SkSource::kStream);
+                           optional_split || x_kind != 1 ? SkSource::kOptional : SkSource::kStream);
 }
 
 hipError_t launch_shared_linear_noalloc(const void* x0, int m0, const void* x1, int m1,

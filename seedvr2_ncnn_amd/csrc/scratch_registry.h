@@ -62,6 +62,18 @@ public:
         return 0;
     }
 
+    // The entry if there is one, else *out null; makes no runtime call but for
+    // the device's number.
+    int find(int kind, void* stream, size_t bytes, void** out) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        int dev = 0;
+        int ret = ops_.current_device(&dev);
+        if (ret != 0) return ret;
+        Map::iterator it = map_.find(Key(dev, kind, stream));
+        *out = it == map_.end() ? 0 : it->second.ptr;
+        return *out && it->second.bytes != bytes ? kMisuse : 0;
+    }
+
     int release(int kind, void* stream) {
         std::lock_guard<std::mutex> lock(mutex_);
         int dev = 0;

@@ -39,6 +39,25 @@ hipError_t stream_scratch(ScratchKind kind, hipStream_t stream, size_t bytes, vo
     return as_hip(registry().get((int)kind, stream, bytes, out));
 }
 
+hipError_t stream_scratch_optional(ScratchKind kind, hipStream_t stream, size_t bytes, void** out) {
+    if ((int)kind < 0 || (int)kind >= kScratchKinds) return hipErrorInvalidValue;
+    const hipError_t e = as_hip(registry().find((int)kind, stream, bytes, out));
+    if (e != hipSuccess || *out) return e;
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess ||
+        status != hipStreamCaptureStatusNone || hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return hipSuccess;
+    }
+    if (registry().get((int)kind, stream, bytes, out) != 0) {
+        (void)hipGetLastError();
+        *out = nullptr;
+    }
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return hipSuccess;
+}
+
 hipError_t stream_scratch_acquire(hipStream_t stream) {
     for (int kind = 0; kind < kScratchKinds; kind++) {
         size_t bytes = 0;

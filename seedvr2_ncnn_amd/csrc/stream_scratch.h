@@ -25,6 +25,11 @@ enum ScratchKind {
 // request of one kind must ask for the same size.
 hipError_t stream_scratch(ScratchKind kind, hipStream_t stream, size_t bytes, void** out);
 
+// The same for a caller that can do without: *out is null where the scratch
+// does not exist yet and cannot be made now, on a capturing stream or for want
+// of memory.  Another thread's capture of another stream is not disturbed.
+hipError_t stream_scratch_optional(ScratchKind kind, hipStream_t stream, size_t bytes, void** out);
+
 // One owner reference to every kind of scratch of (current device, stream),
 // made and zeroed on the stream now if it does not exist yet; released by
 // stream_scratch_release, whose last call waits for the stream and frees it.

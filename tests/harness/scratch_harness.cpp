@@ -71,6 +71,12 @@ int hs_get(int kind, long stream, long bytes, long* out) {
     *out = (long)p;
     return ret;
 }
+int hs_find(int kind, long stream, long bytes, long* out) {
+    void* p = 0;
+    const int ret = g_reg->find(kind, (void*)stream, (size_t)bytes, &p);
+    *out = (long)p;
+    return ret;
+}
 int hs_owners(int kind, long stream) { return g_reg->owners(kind, (void*)stream); }
 // Copies the call log (and clears it); returns its length.
 int hs_take_log(char* buf, int cap) {

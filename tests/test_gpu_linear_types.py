@@ -32,3 +32,29 @@ def test_equals_the_rounded_activations_as_bf16(mv, mt, k, n, act):
         torch.cuda.synchronize()
         assert torch.equal(got[0], ref[0])
         assert not mt or torch.equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+def test_capture_on_a_stream_that_nobody_owns(dtype):
+    """A shape whose tail is split, captured before any call on the stream: the
+    call needs no scratch there (none can be made under capture) and every
+    replay is the rounded operands' product within the bound of an fp32 sum of k
+    products, (k + 2) 2^-24 of the sum of their magnitudes."""
+    import torch
+    mv, k, n = 300, 2560, 1000
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    draw = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    x, w, b = draw(mv, k).to(getattr(torch, dtype)), (0.02 * draw(n, k)).bfloat16(), 0.02 * draw(n)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        y, _ = capi.shared_linear(x, None, w, b, out_dtype=torch.float32)
+    wd = w.double().t().contiguous()
+    for i in range(3):
+        x.copy_(draw(mv, k))
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        xd = x.bfloat16().double()
+        bound = (k + 2) * 2.0 ** -24 * (xd.abs() @ wd.abs() + b.abs().double())
+        assert ((y.double() - (xd @ wd + b.double())).abs() <= bound).all()

@@ -36,6 +36,7 @@ def reg():
     L.hs_acquire.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_long]
     L.hs_release.argtypes = [ctypes.c_int, ctypes.c_long]
     L.hs_get.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_long, ctypes.POINTER(ctypes.c_long)]
+    L.hs_find.argtypes = L.hs_get.argtypes
     L.hs_owners.argtypes = [ctypes.c_int, ctypes.c_long]
     L.hs_take_log.argtypes = [ctypes.c_char_p, ctypes.c_int]
     L.hs_reset()
@@ -124,6 +125,18 @@ def test_a_size_mismatch_and_a_failed_allocation_are_errors(reg):
     assert reg.hs_owners(0, 3) == -1                    # nothing half-made is left
     reg.hs_fail_alloc(0)
     assert reg.hs_acquire(0, 3, MB64) == 0
+
+
+def test_find_makes_nothing(reg):
+    out = ctypes.c_long(5)
+    assert reg.hs_find(0, 7, MB64, ctypes.byref(out)) == 0 and out.value == 0
+    assert _log(reg) == [] and reg.hs_owners(0, 7) == -1
+    assert reg.hs_acquire(0, 7, MB64) == 0
+    p = int(_log(reg)[0][1])
+    assert reg.hs_find(0, 7, MB64, ctypes.byref(out)) == 0 and out.value == p
+    assert reg.hs_find(0, 8, MB64, ctypes.byref(out)) == 0 and out.value == 0
+    assert reg.hs_find(0, 7, 1024, ctypes.byref(out)) == -1
+    assert _log(reg) == [] and reg.hs_owners(0, 7) == 1
 
 
 def _code_lines(path):
