@@ -333,23 +333,34 @@ __global__ void __launch_bounds__(kThreads) cfg_kernel(const float* __restrict__
     }
 }
 
-// Pass 2 of apply_cfg: cfg *= factor, skipped when std(cfg) was 0.
+// Pass 2 of apply_cfg: cfg *= factor, skipped when std(cfg) was 0.  A block
+// takes runs of 1024 elements, gridDim.x apart, behind one factor: joining the
+// records costs it up to 40 KB of reads, five times a run's own 8 KB.  With a
+// run a block, 16 M elements took 87 us in both passes and 50 M 281 (87 and 224
+// with the records joined once, in the statistics pass); so they take 58 and 188.
+constexpr int kScaleBlocks = 2048;   // eight workgroups a CU: every wave slot
 __global__ void __launch_bounds__(kThreads) cfg_scale_kernel(float* __restrict__ out, long count,
                                                              const CfgScratch* sc, int nrec,
                                                              float rescale) {
 #pragma clang fp contract(off)
     __shared__ double red[8];
-    const long i = ((long)blockIdx.x * kThreads + threadIdx.x) * 4;
+    const long step = (long)gridDim.x * (kThreads * 4);
+    long i = ((long)blockIdx.x * kThreads + threadIdx.x) * 4;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (i + 3 < count) v = *reinterpret_cast<const float4*>(out + i);
     float f;
     if (!cfg_factor(sc, nrec, count, rescale, red, &f)) return;
-    if (i + 3 < count) {
+    while (i + 3 < count) {
+        // the next run's load goes out before this one's store
+        const long j = i + step;
+        float4 next = v;
+        if (j + 3 < count) next = *reinterpret_cast<const float4*>(out + j);
         v.x *= f, v.y *= f, v.z *= f, v.w *= f;
         *reinterpret_cast<float4*>(out + i) = v;
-    } else {
-        for (long e = i; e < count; ++e) out[e] *= f;
+        v = next;
+        i = j;
     }
+    for (long e = i; e < count; ++e) out[e] *= f;   // the thread with the ragged end
 }
 
 // ---- Euler update (seedvr2_pipeline.cpp:575-588) ----------------------------
@@ -544,7 +555,8 @@ hipError_t launch_cfg(const float* pos, const float* neg, long count, float scal
     if (e != hipSuccess) return e;
     e = launch_stats(pos, neg, count, scale, out, sc, stream);
     if (e != hipSuccess) return e;
-    cfg_scale_kernel<<<grid, kThreads, 0, stream>>>(out, count, sc, stat_blocks(count), rescale);
+    cfg_scale_kernel<<<min(grid, (unsigned)kScaleBlocks), kThreads, 0, stream>>>(
+        out, count, sc, stat_blocks(count), rescale);
     return hipGetLastError();
 }
 

@@ -111,6 +111,20 @@ def test_apply_cfg(count, scale, rescale):
         assert float(rel.max()) <= 3e-7
 
 
+# ragged counts past 2048 runs of the scaling pass, past 512 records, past the
+# most records (1024, a block's second chunk), and past three runs a block
+@pytest.mark.parametrize("count", [2048 * 1024 + 5, 700 * 4096 + 3, 1024 * 4096 + 4099,
+                                   3 * 2048 * 1024 + 1021])
+def test_apply_cfg_many_elements(count):
+    g = np.random.default_rng(count)
+    pos = g.standard_normal(count).astype(np.float32)
+    neg = (0.8 * pos + 0.3 * g.standard_normal(count)).astype(np.float32)
+    ref = oracle.apply_cfg(pos, neg, 6.5, 0.7)
+    got = _host(capi.apply_cfg(_cuda(pos), _cuda(neg), 6.5, 0.7))
+    rel = np.abs(got - ref) / np.maximum(np.abs(ref), 1e-30)
+    assert float(rel.max()) <= 3e-7
+
+
 def test_apply_cfg_zero_spread_and_nan():
     pos = np.full(5000, 2.0, np.float32)
     neg = np.full(5000, 1.0, np.float32)
