@@ -10,8 +10,8 @@ from seedvr2_ncnn_amd import capi
 pytestmark = pytest.mark.gpu
 
 # one row; a video tail off an 8-row group with text rows in its tile; two,
-# four and six 32-k steps (the pipeline's start and end); ragged n (direct
-# stores); a split tail; rows past two tiles
+# four and six 32-k steps (the pipeline's start and end); n that ends inside a
+# wave's columns; a split tail; rows past two tiles
 CASES = [(1, 0, 64, 64), (37, 5, 128, 40), (250, 70, 192, 260), (257, 3, 64, 512),
          (300, 40, 2560, 1000), (600, 1, 1088, 2560)]
 
@@ -32,6 +32,31 @@ def test_equals_the_rounded_activations_as_bf16(mv, mt, k, n, act):
         torch.cuda.synchronize()
         assert torch.equal(got[0], ref[0])
         assert not mt or torch.equal(got[1], ref[1])
+
+
+# n that no 16-byte row piece covers (7: direct stores in every type; 12: in the
+# 16-bit ones), one 16-byte piece, and a split tail
+@pytest.mark.parametrize("mv,mt,k,n", [(37, 5, 128, 7), (130, 3, 192, 12), (257, 3, 64, 8),
+                                       (300, 40, 2560, 1000)])
+@pytest.mark.parametrize("dtype", ["float32", "float16"])
+def test_outputs_bias_and_entry_points(mv, mt, k, n, dtype):
+    """Every output type, with and without a bias, through both entry points: the
+    bits of the rounded activations given as bf16, and 16-bit outputs the
+    rounding of the fp32 one."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    draw = lambda *s: torch.randn(*s, generator=gen, device="cuda")
+    dt = getattr(torch, dtype)
+    xs = [draw(mv, k).to(dt), draw(mt, k).to(dt)]
+    w, b = (0.02 * draw(n, k)).bfloat16(), 0.02 * draw(n)
+    for bias in (b, None):
+        full = capi.shared_linear(*xs, w, bias, out_dtype=torch.float32)
+        for odt in (torch.float32, torch.bfloat16, torch.float16):
+            ref = capi.shared_linear(*[x.bfloat16() for x in xs], w, bias, out_dtype=odt)
+            for noalloc in (False, True):
+                got = capi.shared_linear(*xs, w, bias, out_dtype=odt, noalloc=noalloc)
+                for y, r, f in zip(got, ref, full):
+                    assert torch.equal(y, r) and torch.equal(y, f.to(odt))
 
 
 @pytest.mark.parametrize("dtype", ["float32", "float16"])

@@ -2,10 +2,13 @@
 MultiHeadAttention over one blob) against the CPU oracle.
 
 The device runs the projections and both attention products in bf16 with
-fp32 accumulation (scores stay fp32 until the softmax, probabilities are
-rounded to bf16).  The bar is the path's: max-abs <= 2e-2 and cosine >=
+fp32 accumulation (scores and exponentials are formed in fp32; the weights of V
+are rounded to bf16, and in long sequences divided by their sum afterwards).  The
+bar is the path's: max-abs <= 2e-2 and cosine >=
 0.9999 against the fp32-input oracle.  Sequences of VAE size are checked on
 a spread of query rows (the oracle computes only those rows)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -96,12 +99,13 @@ def _reference_weights(g, kind, heads):
     """64 channels a head.  plain: scores near zero.  shifted: q and k share a
     constant channel of 40, so every score is near 200 and the exponentials
     need a reference.  general: q's constant channel is another than k's, so
-    the scores are near zero but far below |q| |k| and no reference shows it."""
+    the scores are near zero but far below |q| |k| and no reference shows it.
+    kind may name one of these per head."""
     e = 64 * heads
     ws = _weights(g, e, e)
-    if kind != "plain":
-        for h in range(heads):
-            for i, c in ((0, 0), (2, 0 if kind == "shifted" else 1)):
+    for h, of_head in enumerate([kind] * heads if isinstance(kind, str) else kind):
+        if of_head != "plain":
+            for i, c in ((0, 0), (2, 0 if of_head == "shifted" else 1)):
                 for ch in (0, 1):
                     ws[i][64 * h + ch] = 0
                     ws[i + 1][64 * h + ch] = 40 if ch == c else 0
@@ -164,6 +168,48 @@ def test_mha_large_and_small_values(const, same, size):
     ws[6] = (ws[6] / size).astype(np.float32)
     rows = np.arange(0, 1100, 37).astype(np.int32)
     assert_close(_run(_device(1, ws), x)[rows], oracle.mha(x, 1, *ws, rows=rows, threads=16))
+
+
+@pytest.mark.parametrize("kinds", [("general", "plain"), ("plain", "general"),
+                                   ("shifted", "general", "plain"), ("general", "shifted")])
+def test_mha_heads_of_different_kinds(kinds):
+    """The flag, the row sums and the row scale are one head's at a time: what a
+    head leaves in them must not reach the next one.  The output projection
+    keeps the heads' channels apart, so each is compared by itself."""
+    seq, heads = 4096, len(kinds)
+    g = np.random.default_rng(sum(map(len, kinds)))
+    x = g.standard_normal((seq, 64 * heads)).astype(np.float32)
+    ws = _reference_weights(g, kinds, heads)
+    ws[6] *= np.kron(np.eye(heads), np.ones((64, 64))).astype(np.float32) * np.sqrt(heads)
+    got = _run(_device(heads, ws), x)
+    rows = np.arange(0, seq, 151).astype(np.int32)
+    ref = oracle.mha(x, heads, *ws, rows=rows, threads=16, fast=True)
+    for h in range(heads):
+        assert_close(got[rows, 64 * h:64 * h + 64], ref[:, 64 * h:64 * h + 64])
+
+
+@pytest.mark.parametrize("seq,heads", [(64, 1), (320, 2), (1024, 1), (4096, 2)])
+def test_mha_bf16_rows_read_in_place(seq, heads):
+    """bf16 rows that need no padding are not staged: the same bits as for the
+    same values given as fp32 (which are), x as it was, also with out = x."""
+    import torch
+    g = np.random.default_rng(seq)
+    e = 64 * heads
+    mha = _device(heads, _weights(g, e, e))
+    x = torch.from_numpy(g.standard_normal((seq, e)).astype(np.float32)).cuda().bfloat16()
+    kept = x.clone()
+    ref = mha.forward(x.float(), out_dtype=torch.bfloat16)
+    got = mha.forward(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref) and torch.equal(x, kept)
+    ptr, n = ctypes.byref(mha.config), ctypes.c_size_t()
+    capi.check(capi.lib().s2_mha_workspace_bytes(ptr, seq, ctypes.byref(n)))
+    work = torch.empty(n.value, dtype=torch.uint8, device="cuda")
+    capi.check(capi.lib().s2_mha_forward(
+        ptr, mha.prepared.data_ptr(), x.data_ptr(), capi.DTYPE_BF16, seq, x.data_ptr(),
+        capi.DTYPE_BF16, work.data_ptr(), n.value, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(x, ref)
 
 
 def test_mha_long_sequence_nan_reaches_every_row():
