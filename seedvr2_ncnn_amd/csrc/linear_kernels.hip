@@ -335,6 +335,11 @@ __device__ __forceinline__ void stage_rows4(uint8_t* p, int pitch, const float (
 //   kActRowScale  y = acc * (scale of the row) + bias
 constexpr int kActExp = 100, kActRowScale = 101;
 
+// How the plain epilogues store a wave's staged rows: 16-byte chunks of rows
+// whose pitch is a multiple of 64 bytes, non-temporal; of other rows, by way of
+// the L2; or single elements, where chunks would not keep to the rows.
+enum : int { kWholeSectors, kPieces, kElements };
+
 // XK is the element type of x0 and x1 (0 fp32, 1 bf16, 2 fp16).
 template <int YK, int ACT, int AWA = 0, int RES = 0, int XK = 1>
 __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
@@ -448,7 +453,14 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // past n (an offset with bit 31 set: offsets are below 2^31, the launcher
     // checks 256 rows of output), without a branch per store; the 8 rows of a
     // store lie in one stream.  The output is not read again by this launch:
-    // the stores are non-temporal, leaving the L2 to the operand tiles.
+    // the stores are non-temporal, leaving the L2 to the operand tiles, where
+    // row pitches are multiples of 64 bytes.  Elsewhere the pieces of two waves
+    // meet inside a 64-byte sector, which the L2 has to put together: 9000 x 64 by
+    // 9000 x 64 took 84 us with non-temporal stores, 51 by way of the L2 (62 from
+    // 512-byte rows); 21664 x 2560 by 3112 x 2560 287 and 285.  Rows of n % 8 != 0
+    // leave as elements, 64 columns of a row a store: 3677 x 2560 by 2561 x 2560
+    // 67 us straight from the accumulators (16 columns of a row), 51 so; 4609 x
+    // 512 by 4609 x 512 67 and 36.
     auto wave_epilogue = [&]() {
         if constexpr (YK != 0 && AWA == 0 && RES == 0 && ACT != S2_ACT_SWIGLU) {
             const EpiIds ei = epi_ids();
@@ -525,8 +537,33 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                     const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
                     bv[j] = (bias && col < n) ? bias[col] : 0.f;
                 }
-                const int cb = col0 + ei.wn * 64 + (ln & 7) * 8;   // the lane's 16-byte chunk
+                const int cw = col0 + ei.wn * 64;     // the wave's first column
+                const int cb = cw + (ln & 7) * 8;     // the lane's 16-byte chunk
                 const uint32_t drop = cb < ny ? 0u : 0x80000000u;
+                const uint32_t drop1 = cw + ln < ny ? 0u : 0x80000000u;
+                auto store = [&](auto mode, const uint8_t* buf, int r0) {
+                    constexpr int MODE = decltype(mode)::value;
+                    constexpr int POLICY = MODE == kWholeSectors ? kNonTemporal : 0;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {   // eight rows, of one stream
+                        const __amdgpu_buffer_rsrc_t rs = row0 + r0 + 8 * r < mv ? rs0 : rs1;
+                        if constexpr (MODE == kElements) {
+#pragma unroll
+                            for (int i = 0; i < 8; ++i)
+                                __builtin_amdgcn_raw_buffer_store_b16(
+                                    *(const uint16_t*)(buf + (8 * r + i) * RP + ln * 2), rs,
+                                    (uint32_t)((r0 + 8 * r + i) * pitch + (cw + ln) * 2) | drop1, 0, POLICY);
+                        } else {
+                            __builtin_amdgcn_raw_buffer_store_b128(
+                                *(const u32x4*)(buf + (8 * r + (ln >> 3)) * RP + (ln & 7) * 16), rs,
+                                (uint32_t)((r0 + 8 * r + (ln >> 3)) * pitch + cb * 2) | drop, 0, POLICY);
+                        }
+                    }
+                };
+                // (row scales come with whole chunks: linear_rows)
+                const int mode = ACT != kActRowScale && (ny & 7) != 0 ? kElements
+                                 : pitch % 64 == 0                    ? kWholeSectors
+                                                                      : kPieces;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     uint8_t* buf = mine + (c & 1) * 32 * RP;
@@ -550,15 +587,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                         }
                     }
                     asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const u32x4 sv = *(const u32x4*)(buf + (8 * r + (ln >> 3)) * RP + (ln & 7) * 16);
-                        const uint32_t off = (uint32_t)((r0 + 8 * r + (ln >> 3)) * pitch + cb * 2) | drop;
-                        if (row0 + r0 + 8 * r < mv)
-                            __builtin_amdgcn_raw_buffer_store_b128(sv, rs0, off, 0, kNonTemporal);
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b128(sv, rs1, off, 0, kNonTemporal);
-                    }
+                    if (mode == kWholeSectors)
+                        store(std::integral_constant<int, kWholeSectors>{}, buf, r0);
+                    else if (mode == kPieces)
+                        store(std::integral_constant<int, kPieces>{}, buf, r0);
+                    else
+                        store(std::integral_constant<int, kElements>{}, buf, r0);
                     asm volatile("" ::: "memory");
                 }
             }
@@ -1146,9 +1180,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         }
     };
 
-    // fp32 outputs in whole 16-byte chunks, as in wave_epilogue: a wave's rows
-    // leave 16 at a time, 256 bytes of 4 rows a store (in two halves of 128
-    // whole rows before: 3677 x 2560 by 2560 x 2560 from fp32 104 us, 101 so).
+    // fp32 outputs, as in wave_epilogue: a wave's rows leave 16 at a time, 256
+    // bytes of 4 rows a store (in two halves of 128 whole rows before: 3677 x 2560
+    // by 2560 x 2560 from fp32 104 us, 101 so), or of one row where n % 4 != 0 (4609
+    // x 512 by 4609 x 512 65 us straight from the accumulators, 40 so).
     auto wave_epilogue_f32 = [&]() {
         if constexpr (YK == 0 && AWA == 0 && RES == 0 && ACT != S2_ACT_SWIGLU) {
             const EpiIds ei = epi_ids();
@@ -1169,8 +1204,30 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                 const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
                 bv[j] = (bias && col < n) ? bias[col] : 0.f;
             }
-            const int cb = col0 + ei.wn * 64 + (ln & 15) * 4;   // the lane's 16-byte chunk
+            const int cw = col0 + ei.wn * 64;      // the wave's first column
+            const int cb = cw + (ln & 15) * 4;     // the lane's 16-byte chunk
             const uint32_t drop = cb < n ? 0u : 0x80000000u;
+            const uint32_t drop1 = cw + ln < n ? 0u : 0x80000000u;
+            auto store = [&](auto mode, const uint8_t* buf, int r0) {
+                constexpr int MODE = decltype(mode)::value;
+                constexpr int POLICY = MODE == kWholeSectors ? kNonTemporal : 0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {   // four rows, of one stream
+                    const __amdgpu_buffer_rsrc_t rs = row0 + r0 + 4 * r < mv ? rs0 : rs1;
+                    if constexpr (MODE == kElements) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            __builtin_amdgcn_raw_buffer_store_b32(
+                                *(const uint32_t*)(buf + (4 * r + i) * RP + ln * 4), rs,
+                                (uint32_t)((r0 + 4 * r + i) * pitch + (cw + ln) * 4) | drop1, 0, POLICY);
+                    } else {
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            *(const u32x4*)(buf + (4 * r + (ln >> 4)) * RP + (ln & 15) * 16), rs,
+                            (uint32_t)((r0 + 4 * r + (ln >> 4)) * pitch + cb * 4) | drop, 0, POLICY);
+                    }
+                }
+            };
+            const int mode = (n & 3) != 0 ? kElements : pitch % 64 == 0 ? kWholeSectors : kPieces;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 uint8_t* buf = mine + (i & 1) * 16 * RP;
@@ -1184,15 +1241,12 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
                         *(float*)(buf + (4 * ei.g + r) * RP + (16 * j + ei.l16) * 4) = v;
                     }
                 asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const u32x4 sv = *(const u32x4*)(buf + (4 * r + (ln >> 4)) * RP + (ln & 15) * 16);
-                    const uint32_t off = (uint32_t)((r0 + 4 * r + (ln >> 4)) * pitch + cb * 4) | drop;
-                    if (row0 + r0 + 4 * r < mv)
-                        __builtin_amdgcn_raw_buffer_store_b128(sv, rs0, off, 0, kNonTemporal);
-                    else
-                        __builtin_amdgcn_raw_buffer_store_b128(sv, rs1, off, 0, kNonTemporal);
-                }
+                if (mode == kWholeSectors)
+                    store(std::integral_constant<int, kWholeSectors>{}, buf, r0);
+                else if (mode == kPieces)
+                    store(std::integral_constant<int, kPieces>{}, buf, r0);
+                else
+                    store(std::integral_constant<int, kElements>{}, buf, r0);
                 asm volatile("" ::: "memory");
             }
         }
@@ -1342,32 +1396,10 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             wave_residual();
             return;
         }
-        if (YK && (ny & 7) == 0) {
+        if constexpr (YK != 0)
             wave_epilogue();
-            return;
-        }
-        if (!YK && (n & 3) == 0) {
+        else
             wave_epilogue_f32();
-            return;
-        }
-        const EpiIds ei = epi_ids();
-        // ragged n: direct stores
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = col0 + ei.wn * 64 + 16 * j + ei.l16;
-            if (col >= n) continue;
-            const float bv = bias ? bias[col] : 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    void* yr = out_row(ei.wm * 128 + 16 * i + 4 * ei.g + r);
-                    if (!yr) continue;
-                    float v = acc[i][j][r] + bv;
-                    if (ACT == S2_ACT_GELU) v = gelu(v);
-                    store1<YK>(yr, col, v);
-                }
-        }
     };
 
     // Work of this workgroup as segments (tile, k-iterations [kb, ke)).  A
@@ -1407,8 +1439,7 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
         bool finish = kb == 0 && ke == nk;
         // a whole tile whose waves write their own parts: no wave meets
         // another after the last MFMA phase, so the barrier there is left out
-        const bool free = AWA == 0 && XK == 1 && ACT != S2_ACT_SWIGLU && finish &&
-                          (RES != 0 || (YK ? (ny & 7) == 0 : (n & 3) == 0));
+        const bool free = AWA == 0 && XK == 1 && ACT != S2_ACT_SWIGLU && finish;
         if constexpr (XK == 1)
             mainloop(kb, ke, free);
         else

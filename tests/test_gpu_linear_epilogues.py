@@ -24,8 +24,10 @@ def _inputs(mv, mt, k, n):
 
 
 @pytest.mark.parametrize("mv,mt", ROWS)
-@pytest.mark.parametrize("n", COLS + [12, 7])
+@pytest.mark.parametrize("n", COLS + [12, 7, 288, 261])
 def test_plain_outputs(mv, mt, n):
+    # (rows of whole 64-byte sectors: 288; of 16-byte chunks that share sectors:
+    # COLS, and 12 in fp32; of single elements: 12 in 16 bits, 7, 261)
     import torch
     k = 128
     _, xv, xt, w, b = _inputs(mv, mt, k, n)
