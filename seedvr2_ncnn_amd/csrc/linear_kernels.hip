@@ -1258,6 +1258,15 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
     // x: each element is read and written by one lane.  (Assembled over a
     // workgroup and loaded in two halves before: MLP of 1485 rows 216 us, 210
     // so; of the 720p video 1816 and 1803.)
+    //
+    // A wave goes over its part once for each (stream, sample) that it has rows
+    // of, nearly always one, behind descriptors that end with those rows: the
+    // gate, the descriptor and the residual's type are then fixed for straight
+    // code, where the loads of a quarter are waited for without the stores issued
+    // since.  With their branches in every row a launch of few tiles, which
+    // nothing else hides, took 14 us longer: 64 rows of 2560 to 2560 50.1 us (40.2
+    // assembled over a workgroup), 33.8 so; 1549 rows of 10240 to 2560 109 and 98,
+    // 21,664 rows 879 and 854.
     auto wave_residual = [&]() {
         if constexpr (RES != 0) {
 #pragma clang fp contract(off)
@@ -1265,119 +1274,114 @@ __global__ __launch_bounds__(512, 1) void shared_linear_256_kernel(
             const int ln = ei.tid & 63;
             constexpr int RP = 64 * 2 + 16;   // staged row (bytes)
             uint8_t* mine = lds + (ei.wm * 4 + ei.wn) * kWaveStage;
-            const int es = res.x_kind == 0 ? 4 : 2;
-            const int pitch = n * es;
-            const int rows0 = max(min(m0 - row0, BM), 0);
-            const int rows1 = row0 + BM > mv ? min(mv + m1 - row0, BM) : 0;
-            const __amdgpu_buffer_rsrc_t rx0 = __builtin_amdgcn_make_buffer_rsrc(
-                (char*)res.x[0] + (long)row0 * pitch, (short)0, rows0 * pitch, kRawBufferFormat);
-            const __amdgpu_buffer_rsrc_t rx1 = __builtin_amdgcn_make_buffer_rsrc(
-                (char*)res.x[1] + (long)(row0 - mv) * pitch, (short)0, rows1 * pitch, kRawBufferFormat);
-            const __amdgpu_buffer_rsrc_t ro0 = __builtin_amdgcn_make_buffer_rsrc(
-                (char*)res.out[0] + (long)row0 * pitch, (short)0, rows0 * pitch, kRawBufferFormat);
-            const __amdgpu_buffer_rsrc_t ro1 = __builtin_amdgcn_make_buffer_rsrc(
-                (char*)res.out[1] + (long)(row0 - mv) * pitch, (short)0, rows1 * pitch, kRawBufferFormat);
+            const int wrow = row0 + 128 * ei.wm;   // the wave's first row
             const int sub = ln >> 4;
             const int col = col0 + ei.wn * 64 + (ln & 15) * 4;   // n is a multiple of 8
             const bool in = col < n;
-            const uint32_t drop = in ? 0u : 0x80000000u;
             float bv[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int c = col0 + ei.wn * 64 + 16 * j + ei.l16;
                 bv[j] = (bias && c < n) ? bias[c] : 0.f;
             }
-            // 8-byte chunks of 16-bit residuals come in the first two words
-            auto load = [&](int c, u32x4 (&raw)[8]) {
+            // rows [l, e) of the stream, which lies `at` rows above the wave
+            auto segment = [&](auto kind, const void* x, void* out, f32x4 g, int at, int l, int e) {
+                constexpr int KIND = decltype(kind)::value;
+                constexpr int ES = KIND == 0 ? 4 : 2;
+                typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+                typedef typename std::conditional<KIND == 0, u32x4, u32x2>::type Raw;   // four columns
+                const int pitch = n * ES;
+                const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+                    (char*)const_cast<void*>(x) + (long)l * pitch, (short)0, (e - l) * pitch, kRawBufferFormat);
+                const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+                    (char*)out + (long)l * pitch, (short)0, (e - l) * pitch, kRawBufferFormat);
+                // (rows above l have negative offsets, which are past the end too;
+                // a column past n starts half the range away, so that no row's
+                // offset brings it back)
+                const uint32_t off = in ? (uint32_t)((at + sub - l) * pitch + col * ES) : 0x80000000u;
+                auto load = [&](int c, Raw (&raw)[8]) {
 #pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int rl = ei.wm * 128 + 32 * c + 4 * r;
-                    const uint32_t off = (uint32_t)((rl + sub) * pitch + col * es) | drop;
-                    const bool video = row0 + rl < mv;   // 8-row groups lie in one stream
-                    if (res.x_kind == 0) {
-                        raw[r] = video ? __builtin_amdgcn_raw_buffer_load_b128(rx0, off, 0, kNonTemporal)
-                                       : __builtin_amdgcn_raw_buffer_load_b128(rx1, off, 0, kNonTemporal);
-                    } else {
-                        const auto h = video ? __builtin_amdgcn_raw_buffer_load_b64(rx0, off, 0, kNonTemporal)
-                                             : __builtin_amdgcn_raw_buffer_load_b64(rx1, off, 0, kNonTemporal);
-                        raw[r][0] = h[0];
-                        raw[r][1] = h[1];
+                    for (int r = 0; r < 8; ++r) {
+                        const int so = (32 * c + 4 * r) * pitch;
+                        if constexpr (KIND == 0)
+                            raw[r] = __builtin_amdgcn_raw_buffer_load_b128(rx, off + so, 0, kNonTemporal);
+                        else
+                            raw[r] = __builtin_amdgcn_raw_buffer_load_b64(rx, off + so, 0, kNonTemporal);
                     }
+                };
+                Raw raw[2][8];
+                load(0, raw[0]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    if (c < 3) load(c + 1, raw[(c + 1) & 1]);
+                    uint8_t* buf = mine + (c & 1) * 32 * RP;
+#pragma unroll
+                    for (int ii = 0; ii < 2; ++ii)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            float v[4];
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) v[r] = acc[2 * c + ii][j][r] + bv[j];
+                            stage_rows4<1>(buf + (16 * ii + 4 * ei.g) * RP + (16 * j + ei.l16) * 2, RP, v);
+                        }
+                    asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) {
+                        const Raw xr = raw[c & 1][r];
+                        const uint2 yw = *(const uint2*)(buf + (4 * r + sub) * RP + (ln & 15) * 8);
+                        float o[4];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const uint16_t hv = (uint16_t)(xr[i >> 1] >> (16 * (i & 1)));
+                            const float xf = KIND == 0   ? __uint_as_float(xr[KIND == 0 ? i : 0])
+                                             : KIND == 1 ? bf16_to_f32(hv)
+                                                         : (float)__builtin_bit_cast(_Float16, hv);
+                            const uint32_t w = i >> 1 ? yw.y : yw.x;
+                            const float y = __uint_as_float(i & 1 ? (w & 0xffff0000u) : (w << 16));
+                            const float p = y * g[i];
+                            o[i] = xf + p;
+                        }
+                        const int so = (32 * c + 4 * r) * pitch;
+                        if constexpr (KIND == 0) {
+                            const u32x4 ov = {__float_as_uint(o[0]), __float_as_uint(o[1]),
+                                              __float_as_uint(o[2]), __float_as_uint(o[3])};
+                            __builtin_amdgcn_raw_buffer_store_b128(ov, ro, off + so, 0, kNonTemporal);
+                        } else {
+                            const u32x2 ov = KIND == 1
+                                                 ? u32x2{pack2_bf16_rne(o[0], o[1]), pack2_bf16_rne(o[2], o[3])}
+                                                 : u32x2{pack2_f16_rne(o[0], o[1]), pack2_f16_rne(o[2], o[3])};
+                            __builtin_amdgcn_raw_buffer_store_b64(ov, ro, off + so, 0, kNonTemporal);
+                        }
+                    }
+                    asm volatile("" ::: "memory");
                 }
             };
-            int cur = -1;
-            float g[4] = {0.f, 0.f, 0.f, 0.f};
-            u32x4 raw[2][8];
-            load(0, raw[0]);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                if (c < 3) load(c + 1, raw[(c + 1) & 1]);
-                uint8_t* buf = mine + (c & 1) * 32 * RP;
-#pragma unroll
-                for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        float v[4];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) v[r] = acc[2 * c + ii][j][r] + bv[j];
-                        stage_rows4<1>(buf + (16 * ii + 4 * ei.g) * RP + (16 * j + ei.l16) * 2, RP, v);
+#pragma unroll 1
+            for (int stream = wrow < mv ? 0 : 1; stream < 2; ++stream) {
+                const int* ends = res.rows.end + stream * kAdaMaxBatch;
+                const int at = wrow - (stream ? mv : 0);   // the wave's first row, from the stream's
+                const int last = min(at + 128, stream ? m1 : m0);
+                int l = max(at, 0), b = 0;
+#pragma unroll 1
+                while (l < last) {
+                    while (b + 1 < res.rows.batch && l >= ends[b]) ++b;
+                    const int e = b + 1 < res.rows.batch ? min(ends[b], last) : last;
+                    const void* x = stream ? res.x[1] : res.x[0];
+                    void* out = stream ? res.out[1] : res.out[0];
+                    const float* gs = stream ? res.gate_s[1] : res.gate_s[0];
+                    f32x4 g = {0.f, 0.f, 0.f, 0.f};
+                    if (in) {
+                        g = *reinterpret_cast<const f32x4*>(res.gate + (long)b * n + col);
+                        if (gs) g += *reinterpret_cast<const f32x4*>(gs + col);
                     }
-                asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
-#pragma unroll
-                for (int r = 0; r < 8; ++r) {
-                    const int rl = ei.wm * 128 + 32 * c + 4 * r;
-                    const bool video = row0 + rl < mv;
-                    const int local = row0 + rl + sub - (video ? 0 : mv);
-                    // the row's sample: the number of its stream's row ends at
-                    // or below it (the ends are read with uniform indices)
-                    int b = 0;
-                    for (int k2 = 0; k2 + 1 < res.rows.batch; ++k2) {
-                        const int e = video ? res.rows.end[k2] : res.rows.end[kAdaMaxBatch + k2];
-                        if (local >= e) b = k2 + 1;
-                    }
-                    const int key = (video ? 0 : kAdaMaxBatch) + b;
-                    if (key != cur && in) {
-                        cur = key;
-                        const float* ga = res.gate + (long)b * n + col;
-                        const float* gs = video ? res.gate_s[0] : res.gate_s[1];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) g[i] = gs ? ga[i] + gs[col + i] : ga[i];
-                    }
-                    const u32x4 xr = raw[c & 1][r];
-                    const uint2 yw = *(const uint2*)(buf + (4 * r + sub) * RP + (ln & 15) * 8);
-                    float o[4];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint16_t hv = (uint16_t)(xr[i >> 1] >> (16 * (i & 1)));
-                        const float x = res.x_kind == 0   ? __uint_as_float(xr[i])
-                                        : res.x_kind == 1 ? bf16_to_f32(hv)
-                                                          : (float)__builtin_bit_cast(_Float16, hv);
-                        const uint32_t w = i >> 1 ? yw.y : yw.x;
-                        const float y = __uint_as_float(i & 1 ? (w & 0xffff0000u) : (w << 16));
-                        const float p = y * g[i];
-                        o[i] = x + p;
-                    }
-                    const uint32_t off = (uint32_t)((rl + sub) * pitch + col * es) | drop;
-                    if (res.x_kind == 0) {
-                        u32x4 ov;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) ov[i] = __float_as_uint(o[i]);
-                        if (video)
-                            __builtin_amdgcn_raw_buffer_store_b128(ov, ro0, off, 0, kNonTemporal);
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b128(ov, ro1, off, 0, kNonTemporal);
-                    } else {
-                        typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-                        const u32x2 ov = res.x_kind == 1
-                                             ? u32x2{pack2_bf16_rne(o[0], o[1]), pack2_bf16_rne(o[2], o[3])}
-                                             : u32x2{pack2_f16_rne(o[0], o[1]), pack2_f16_rne(o[2], o[3])};
-                        if (video)
-                            __builtin_amdgcn_raw_buffer_store_b64(ov, ro0, off, 0, kNonTemporal);
-                        else
-                            __builtin_amdgcn_raw_buffer_store_b64(ov, ro1, off, 0, kNonTemporal);
-                    }
+                    if (res.x_kind == 0)
+                        segment(std::integral_constant<int, 0>{}, x, out, g, at, l, e);
+                    else if (res.x_kind == 1)
+                        segment(std::integral_constant<int, 1>{}, x, out, g, at, l, e);
+                    else
+                        segment(std::integral_constant<int, 2>{}, x, out, g, at, l, e);
+                    l = e;
                 }
-                asm volatile("" ::: "memory");
             }
         }
     };

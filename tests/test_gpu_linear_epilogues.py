@@ -63,3 +63,33 @@ def test_residual_equals_projection_and_ada_out(mv, mt, n, dtype):
     torch.cuda.synchronize()
     assert torch.equal(got[0], ref[0])
     assert not mt or torch.equal(got[1], ref[1])
+
+
+@pytest.mark.parametrize("mv,mt", ROWS + [(128, 64), (192, 0), (200, 300), (0, 40),
+                                          ((128, 300, 212), (40, 130, 200)),
+                                          ((127, 129, 384), (128, 1, 63)),
+                                          ((500, 0, 140), (64, 0, 64))])
+@pytest.mark.parametrize("n", [8, 264])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("own_gates", [False, True])
+def test_residual_samples_and_streams_of_a_wave(mv, mt, n, dtype, own_gates):
+    """A wave goes over its 128 rows once for each sample of each stream in them:
+    one sample, and three whose ends lie on and off the waves' edges, one of
+    them empty; rows of either stream that fill no wave."""
+    import torch
+    if isinstance(mv, tuple):
+        vr, tr, mv, mt = list(mv), list(mt), sum(mv), sum(mt)
+    else:
+        vr, tr = [mv], [mt] if mt else None
+    draw, xv, xt, w, b = _inputs(mv, mt, 64, n)
+    dt = getattr(torch, dtype)
+    rv, rt = draw(mv, n).to(dt), draw(mt, n).to(dt) if mt else None
+    gate, gates = draw(len(vr), n), dict(video_gate=draw(n), text_gate=draw(n)) if own_gates else {}
+    got = capi.shared_linear_residual(xv, xt, w, b, vr, tr, rv, rt, gate,
+                                      out_video=torch.empty_like(rv),
+                                      out_text=torch.empty_like(rt) if mt else None, **gates)
+    yv, yt = capi.shared_linear(xv, xt, w, b)
+    ref = capi.ada_out(rv.clone(), rt.clone() if mt else None, yv, yt, vr, tr, gate, **gates)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], ref[0])
+    assert not mt or torch.equal(got[1], ref[1])
