@@ -604,7 +604,10 @@ S2_API int s2_vae_pixel_shuffle(const void* packed, s2_dtype dtype, int channels
  * d = embed_dim / num_heads: softmax(scale q_h k_h^T) v_h with q = x Wq^T +
  * bq (likewise k, v), heads concatenated, then out = o Wo^T + bo.  The
  * projections and both attention products run on the matrix cores in bf16
- * with fp32 accumulation; the scores are kept in fp32 until the softmax. */
+ * with fp32 accumulation.  Scores and exponentials are fp32; the weights of v
+ * are rounded to bf16, and divided by the fp32 sum of the rounded weights after
+ * their product with v where the sequence is long (one head from 1,024 tokens,
+ * several from 4,096) and the operands leave room, else before. */
 
 /* ParamDict ids 0, 1 and 6 of the reference load_param (:116-129); qdim =
  * weight_data_size / embed_dim (the input width).  kdim and vdim equal qdim

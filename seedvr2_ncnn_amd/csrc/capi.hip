@@ -108,9 +108,11 @@ struct MhaWork {
 // Sequences from here on take the exponentials in the score product's
 // epilogue, one head (whose q and k come from one product), or several.  The
 // small launches around it cost what the fp32 score matrix and its softmax
-// pass cost at some length: one head of 512, bf16, 256 tokens 104 against 102
-// us, 1024 tokens 112 against 122, 14,400 tokens 540 against 810; with q and k
-// apart 3001 tokens 152 against 151, 4096 tokens 159 against 164.
+// pass cost at some length.  One head of 512, bf16: 1024 tokens 103 against 110
+// us, 14,400 tokens 510 against 741; 512 tokens 92 against 97, which are left
+// with normalised weights.  Eight heads of 64, with q and k apart: 2048 tokens 840
+// against 763 us, 3001 tokens 904 against 964, 4096 tokens 927 against 968, 14,400
+// tokens 2604 against 4721.
 constexpr int kMhaFusedSeq = 1024, kMhaFusedSeqHeads = 4096;
 
 MhaWork mha_work(const s2_mha_config* c, int seq) {
@@ -126,8 +128,8 @@ MhaWork mha_work(const s2_mha_config* c, int seq) {
     w.oh = w.p + align256((size_t)seq * w.lp * 2);
     w.o = w.oh + align256((size_t)seq * d * 2);
     w.total = w.o + (c->num_heads > 1 ? align256((size_t)seq * c->embed_dim * 2) : 0);
-    w.fused = seq >= (c->num_heads == 1 ? kMhaFusedSeq : kMhaFusedSeqHeads) && d % 64 == 0 && (long)256 * w.lp * 4 <= 0x7fffffffL &&
-              (long)512 * d * 4 <= 0x7fffffffL;
+    w.fused = seq >= (c->num_heads == 1 ? kMhaFusedSeq : kMhaFusedSeqHeads) && d % 64 == 0 &&
+              (long)256 * w.lp * 4 <= 0x7fffffffL && (long)512 * d * 4 <= 0x7fffffffL;
     if (w.fused) {
         w.pitch = (seq + 255) / 256 * 256;
         w.parts = 2 * ((seq + 255) / 256);

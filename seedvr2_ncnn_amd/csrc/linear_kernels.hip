@@ -2,9 +2,11 @@
 // y = act(x W^T + b) for the video and the text stream in one grouped launch.
 //
 // x [m][k] and W [n][k] are both k-contiguous, which is the natural operand
-// layout of v_mfma_f32_32x32x16_bf16 (each lane supplies 8 consecutive k of
-// one row of A and one column of B), so both tiles are staged in LDS
-// unchanged.  fp32 activations are rounded to bf16 while they are staged.
+// layout of the bf16 MFMAs (each lane supplies 8 consecutive k of one row of A
+// and one column of B), so both tiles are staged in LDS unchanged.  fp32 and
+// fp16 activations are rounded to bf16 while they are staged.  k that is a
+// multiple of 64 takes the 256x256-tile kernel, other k (and rows too long for
+// its 32-bit offsets) the 128x128 one.
 #include <math.h>
 
 #include <algorithm>
@@ -216,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void shared_linear_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile path for bf16 activations with k % 64 == 0.
+// Large-tile path, k % 64 == 0.
 //
 // Block tile 256x256 with eight waves, two per SIMD, in a 2 (m) x 4 (n) grid
 // of 128x64 wave tiles (8x4 MFMA 16x16x32 accumulators = 128 fp32 per lane).
@@ -231,17 +233,18 @@ __global__ __launch_bounds__(256, 2) void shared_linear_kernel(
 // no VGPR staging).  The buffer descriptors bound each tile to its valid
 // rows, so ragged m and n read zeros.  LDS rows are 128 bytes; 16-byte chunk
 // c of row r is stored at position c ^ (((r >> 1) ^ ((r & 1) << 2)) & 7), so
-// the rows one ds_read_b128 phase touches land on distinct banks.  The bf16
-// epilogue adds the bias and activation in fp32, converts with
-// v_cvt_pk_bf16_f32, assembles the 256x256 tile in LDS and writes it out as
-// 16-byte row chunks.
+// the rows one ds_read_b128 phase touches land on distinct banks.  (That is for
+// bf16 activations; fp32 and fp16 ones have a main loop of their own, which
+// converts A in registers.)  The epilogues add the bias and activation in fp32;
+// each wave converts, stages and stores its own 128x64 part, except for SwiGLU
+// and the fused QKV projection, which assemble the tile in LDS.
 //
 // Tail balancing.  When the tile count leaves the last wave of workgroups
 // partly idle, the tiles of that wave are not given one workgroup each:
 // their 64-k iterations are dealt out evenly to sk_groups workgroups, each
 // taking one contiguous range of (tile, k-iteration) pairs (with sk_groups
-// a multiple of the tile count, every range lies inside one tile).  A tile finished by one workgroup takes the normal epilogue; a tile
-// split between workgroups has every part store its fp32 accumulators to a
+// a multiple of the tile count, every range lies inside one tile).  A tile
+// finished by one workgroup takes the normal epilogue; a tile split between workgroups has every part store its fp32 accumulators to a
 // per-workgroup slot and bump the tile's arrival counter, and the last part
 // to arrive sums all the slots in workgroup order (so the result does not
 // depend on which part arrives last), runs the epilogue and resets the
