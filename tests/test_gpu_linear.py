@@ -44,7 +44,7 @@ def _tight(got, xr, wr, b, act, rows=None):
 
 # the last three put video and text rows in one 256-row tile: the video tail
 # ends off (257, 300) or on (250 -> 256) an 8-row boundary, and n = 260 takes
-# the direct-store epilogue
+# the element stores of the epilogue
 SHAPES = [(1, 0, 8, 16), (37, 5, 24, 40), (130, 64, 72, 136), (64, 64, 128, 2560),
           (257, 3, 2560, 96), (300, 40, 128, 260), (250, 70, 192, 512)]
 
@@ -207,7 +207,7 @@ def test_fp16_activations(mv, mt, k, n, act):
 
 
 # one full wave of 256 tiles (no split tail), a split tail (860 tiles), and an
-# n that is not a multiple of 8 (the direct-store epilogue)
+# n that is not a multiple of 8 (the epilogue's element stores)
 @pytest.mark.parametrize("mv,mt,k,n", [(4000, 64, 256, 4096), (21600, 64, 2560, 2560),
                                        (300, 40, 128, 260)])
 @pytest.mark.parametrize("act", [0, 1])

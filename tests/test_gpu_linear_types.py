@@ -34,7 +34,7 @@ def test_equals_the_rounded_activations_as_bf16(mv, mt, k, n, act):
         assert not mt or torch.equal(got[1], ref[1])
 
 
-# n that no 16-byte row piece covers (7: direct stores in every type; 12: in the
+# n that no 16-byte row piece covers (7: element stores in every type; 12: in the
 # 16-bit ones), one 16-byte piece, and a split tail
 @pytest.mark.parametrize("mv,mt,k,n", [(37, 5, 128, 7), (130, 3, 192, 12), (257, 3, 64, 8),
                                        (300, 40, 2560, 1000)])
